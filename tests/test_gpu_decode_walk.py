@@ -1,0 +1,73 @@
+"""The decode walk's edges against the fp32 oracle: ranges of more page ids
+than the kernel keeps in LDS, rows of a window's first page that lie before
+the window, bias rows at every alignment."""
+from importlib import import_module
+
+import pytest
+import torch
+
+from helpers import assert_lse_close, assert_out_close
+from oracle import attn_ref
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(tm, dev, case, what, rel=None, **kw):
+    ref_o, ref_l = attn_ref.decode_paged(
+        case.q, case.k_pool, case.v_pool, case.block_table, case.ctx_lens,
+        case.scale, window=case.window, rel=rel)
+    c = case.to(dev)
+    out, lse = tm.decode_paged(
+        c.q, c.k_pool, c.v_pool, c.block_table, c.ctx_lens, c.scale,
+        window=c.window, rel=None if rel is None else rel.to(dev), **kw)
+    torch.cuda.synchronize()
+    assert_out_close(out, ref_o, what)
+    assert_lse_close(lse, ref_l, what)
+
+
+@pytest.mark.parametrize("ctx", [[63990, 40], [64017, 1, 0, 33],
+                                 [70, 66000, 65]])
+def test_range_beyond_the_kept_page_ids(tm, dev, ctx):
+    """One work-group walks everything: 4000 page ids are kept without a bias
+    (64,000 tokens), 1500 with one (24,000), the rest are looked up on the
+    way. The last kept page is a step's first or second one, or a sequence's
+    last."""
+    wl = import_module("tm-opt_amd.workloads")
+    g = torch.Generator().manual_seed(41)
+    case = wl.make_decode("ids", 41, len(ctx), 0, 0, hq=4, hkv=1, ctx=ctx)
+    _check(tm, dev, case, f"ids {ctx}", num_workgroups=1)
+    ctx = [max(0, c - 40000) if c > 40000 else c for c in ctx]
+    case = wl.make_decode("ids", 42, len(ctx), 0, 0, hq=4, hkv=1, ctx=ctx)
+    rel = (torch.randn((len(ctx), 4, 300), generator=g) * 0.5).bfloat16()
+    _check(tm, dev, case, f"ids + bias {ctx}", rel, num_workgroups=1)
+
+
+@pytest.mark.parametrize("window", [1, 15, 17, 31, 100])
+def test_window_starts_inside_a_page(tm, dev, window):
+    """Rows of the window's first page that lie before the window hold NaN:
+    they are outside the loads' resource, in K and in V."""
+    wl = import_module("tm-opt_amd.workloads")
+    ctx = [window + k for k in range(0, 34, 3)] + [1, 16, 333]
+    case = wl.make_decode("win", 43, len(ctx), 0, 0, window, ctx=ctx)
+    for b, n in enumerate(ctx):
+        first = max(0, n - window)
+        for p in range(first // 16 * 16, first):
+            page = int(case.block_table[b, p // 16])
+            case.k_pool[page, p % 16] = float("nan")
+            case.v_pool[page, p % 16] = float("nan")
+    _check(tm, dev, case, f"window {window}", min_pages=1)
+
+
+@pytest.mark.parametrize("hq,hkv", [(4, 4), (6, 1), (8, 1), (16, 1), (12, 1),
+                                    (40, 2)])
+@pytest.mark.parametrize("E", [1, 2, 7, 33, 64, 65])
+def test_bias_rows_at_every_alignment(tm, dev, hq, hkv, E):
+    """E odd puts every other row mid-dword; head 0 of sequence 0 starts at
+    the first byte of the tensor, the last head ends at its last one;
+    contexts around E have steps inside, across and past the band."""
+    wl = import_module("tm-opt_amd.workloads")
+    g = torch.Generator().manual_seed(E)
+    ctx = [1, 2, 3, 4, 5, 16, 31, 32, 33, 48, 63, 64, 65, 66, 95, 130]
+    case = wl.make_decode("rel", 44, len(ctx), 0, 0, hq=hq, hkv=hkv, ctx=ctx)
+    rel = torch.randn((len(ctx), hq, E), generator=g).bfloat16()
+    _check(tm, dev, case, f"E={E} {hq}/{hkv}", rel, min_pages=2)

@@ -15,6 +15,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -110,12 +111,96 @@ __device__ __forceinline__ u32x2 lds_ld64(uint32_t addr) {
   return *(const lds_u32x2*)(uintptr_t)addr;
 }
 
+__device__ __forceinline__ uint32_t lds_ld32(uint32_t addr) {
+  return *(const __attribute__((address_space(3))) uint32_t*)(uintptr_t)addr;
+}
+
 // ds_read_b64_tr_b16: within each 16-lane group, lane i receives element
 // i % 4 of the 8-byte chunks addressed by lanes 4j + i / 4 (j = 0..3), i.e.
 // a 4 x 16 block of 16-bit values comes back transposed
 __device__ __forceinline__ bf16x4 lds_tr16(uint32_t addr) {
   return __builtin_bit_cast(
       bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)addr));
+}
+
+// ---- global memory straight into LDS ------------------------------------
+// raw buffer resource: base, byte range, dword 3 as for every buffer access
+// in this library
+// (all fields are wave-uniform; readfirstlane keeps them in scalar
+// registers, as the instruction needs, even where the compiler computed a
+// field with vector instructions)
+__device__ __forceinline__ i32x4 make_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t p = (uint64_t)(uintptr_t)base;
+  return i32x4{__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
+               __builtin_amdgcn_readfirstlane(
+                   (int)((uint32_t)(p >> 32) & 0xffffu)),
+               __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000};
+}
+
+// 16 bytes per lane from global memory straight into LDS: lane l of the
+// wave writes bytes lds + 16 l .. +15. Issued from inline assembly so that
+// the compiler does not wait for it at every barrier or before LDS reads it
+// cannot prove disjoint from it; the kernel waits for these loads itself
+// (wait_vm). The compiler's own waits for ordinary loads (the fused bias)
+// do not count these: they wait for every DMA issued between the load and
+// its use, so the tile loop issues no DMA in that stretch.
+__device__ __forceinline__ void dma(i32x4 rsrc, uint32_t lds, int voff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+      :
+      : "s"(lds), "v"(voff), "s"(rsrc)
+      : "memory", "m0");
+}
+
+// Four of them, 1 KB apart in LDS, non-temporal (data read once: the measured
+// read rate of a plain stream rises from 6.2 to 6.9 TB/s with it). IMM: the
+// steps are the instructions' own offsets, which count for the LDS address and
+// for the memory offset alike (so lane offset i is given less 1024 i, and must
+// not be negative); otherwise M0 moves, and the lane offsets are plain.
+template <bool IMM>
+__device__ __forceinline__ void dma4_nt(i32x4 rsrc, uint32_t lds, int v0,
+                                        int v1, int v2, int v3) {
+  if constexpr (IMM)
+    asm volatile(
+        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %5, 0 offen nt lds\n\t"
+        "buffer_load_dwordx4 %2, %5, 0 offen offset:1024 nt lds\n\t"
+        "buffer_load_dwordx4 %3, %5, 0 offen offset:2048 nt lds\n\t"
+        "buffer_load_dwordx4 %4, %5, 0 offen offset:3072 nt lds"
+        :
+        : "s"(lds), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "s"(rsrc)
+        : "memory", "m0");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %5, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %5, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %3, %5, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %4, %5, 0 offen nt lds"
+        :
+        : "s"(lds), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "s"(rsrc)
+        : "memory", "m0", "scc");
+}
+
+// 4 bytes per lane into LDS: lane l of the wave writes bytes lds + 4 l ..
+// +3 (the fused bias's window rows; the same rules as dma())
+__device__ __forceinline__ void dma32(i32x4 rsrc, uint32_t lds, uint32_t voff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+      :
+      : "s"(lds), "v"(voff), "s"(rsrc)
+      : "memory", "m0");
+}
+
+// wait until at most N vector-memory loads of this wave are in flight
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) |
+                             (15 << 8));
 }
 
 __device__ __forceinline__ void wave_lds_sync() {

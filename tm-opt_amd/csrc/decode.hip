@@ -25,18 +25,25 @@
 //    work-group covers alone is written in place and skipped by the merge.
 //  * One wave per KV head. The four waves of a work-group read the four
 //    256-byte head slices of the same token rows, so together they stream
-//    whole 16 KB pages. K and V arrive by 16-byte buffer loads whose
-//    resource is one page: a missing page (past the range, or a table entry
-//    outside the pool) has zero records, so its loads return zeros without
-//    touching memory, and the next step's loads (query rows included, when
-//    the step starts a new sequence) are always issued before the current
-//    step's math (no branch around them, no vmcnt(0) drain).
+//    whole 16 KB pages.
+//  * K and V go from global memory straight into LDS (buffer_load ... lds,
+//    1 KB per instruction, no registers), per wave into two stages of one
+//    step (two pages, 32 tokens) each. A step's fragments are read into
+//    registers first, which frees its stage for the step after next: two
+//    steps (32 KB per wave) fly while one is computed. The resource of a
+//    load is the rows of one page that hold visible keys: other rows (a
+//    window's first page, a sequence's last one, a missing page, steps past
+//    the range) read as zeros and cost no memory traffic, so every step
+//    issues the same number of loads (no branch around them) and the waits
+//    count exactly.
 //  * Coalesced loads: each group of 16 lanes reads one token's 256-byte
-//    head slice (lanes 16 B apart); the rows are then staged through a
-//    per-wave LDS tile (XOR-swizzled: conflict-free on 64 banks) from which
-//    the MFMA fragments are read, V by transposed reads. Loading the MFMA
-//    layout directly (16 tokens per instruction, lanes 1 KB apart) cost
-//    12-15 % of the bandwidth.
+//    head slice. The tiles are XOR-swizzled (by permuting which 16 bytes a
+//    lane fetches) so that the fragment reads do not conflict on 64 banks;
+//    V^T fragments are transposed reads. Loading the MFMA layout directly
+//    (16 tokens per instruction, lanes 1 KB apart) cost 12-15 % of the
+//    bandwidth.
+//  * The page ids of a work-group's range are fetched before the walk, one
+//    page per thread, into LDS.
 //  * Scores and P.V run on MFMA (v_mfma_f32_16x16x32_bf16). S^T = K.Q^T puts
 //    16 tokens on the M axis and the REP heads (padded to 16) on N, so each
 //    lane owns 8 scores of one head: the running max needs two cross-lane
@@ -46,9 +53,11 @@
 //    read of the pages); a larger one runs as groups of its largest divisor
 //    up to 16, each group a scheduled KV head of its own.
 //
-// Per step (two pages = 32 tokens, tile t = page t):
-//  Load i of tile t brings tokens 16t + 4i + (lane >> 4), 16 bytes (dims
-//  8 (lane & 15)..+7) per lane, into LDS rows of 256 B.
+// What bounds it: HBM on large batches (6.2-6.45 TB/s at 64-128 sequences);
+// on small ones, and beside another kernel, the rate at which one compute
+// unit streams. See the walk for what that rate is made of.
+//
+// Per step (tile t = page t):
 //  S^T: lane (r, g) reads row 16t + r, dims 32kk + 8g..+7 (one 16-byte read).
 //  P.V: the A operand of lane (r, g) is dim 16 blk + r of tokens 4g..4g+3
 //  and 16+4g..16+4g+3 (two transposed reads), matching the P^T lane layout
@@ -64,16 +73,14 @@ constexpr int kD = 128;
 constexpr int kPS = 16;                      // tokens per page
 constexpr int kRowB = 256;                   // one token's head slice
 constexpr int kTileB = 2 * kPS * kRowB;      // 32 tokens: 8 KB
-constexpr int kWaveLds = 2 * kTileB;         // K tile + V tile per wave
-#ifndef TMOPT_DECODE_DEEP
-#define TMOPT_DECODE_DEEP 2
-#endif
-constexpr int kDeep = TMOPT_DECODE_DEEP;     // step ring depth
+constexpr int kBiasB = 5 * 256;              // bias windows of a step, per wave
+// LDS of a wave: two stages of one step each (K tile, V tile, bias windows),
+// then the query rows of a piece
+constexpr int stage_bytes(bool rel) { return 2 * kTileB + (rel ? kBiasB : 0); }
+constexpr int wave_lds(bool rel) { return 2 * stage_bytes(rel) + kPS * kRowB; }
 constexpr int kMaxB = 8192;                  // prefix table lives in LDS
-// cache policy of the K/V page loads: non-temporal (streamed once; the
-// measured read rate of a plain stream rises from 6.2 to 6.9 TB/s with it)
-constexpr int kStreamLoad = 2;
-
+// page ids of a range kept in LDS, beside four waves' tiles
+constexpr int ids_kept(bool rel) { return rel ? 1500 : 4000; }
 struct DecodeArgs {
   const __bf16* q;
   const __bf16* kpool;
@@ -107,6 +114,7 @@ struct DecodeArgs {
   int* geo;          // [B + 2]: C, then the page-stream prefix pref[0..B]
   // read by the REP 0 kernels only (any other REP implies rep == REP,
   // kv_div == 1, HKV_stored == HKV)
+  int ids_off;       // LDS byte offset of the range's page ids
   int rep;           // query heads per scheduled KV head (1..16)
   int kv_div;        // scheduled KV heads per stored one: 1 unless HQ/HKV
                      // is above 16 (then kv_div groups of `rep` query
@@ -124,152 +132,111 @@ __device__ __forceinline__ int vis_pages(int n, int window) {
   return (n + kPS - 1) / kPS - vis_lo(n, window) / kPS;
 }
 
+// The kernel's arguments in the argument segment. `rare`: read again there
+// (the pointer is opaque to the compiler) where they are needed rarely, at a
+// new sequence or a piece's end: held over the walk they cost more scalar
+// registers than there are.
+typedef const __attribute__((address_space(4))) DecodeArgs* ArgsPtr;
+__device__ __forceinline__ ArgsPtr kernel_args(bool rare) {
+  auto p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  if (rare) asm volatile("" : "+s"(p));
+  return p;
+}
+
 // keys of sequence b (its query sits at position n - 1)
 template <int KIND>
-__device__ __forceinline__ int seq_n(const DecodeArgs& a, int b) {
-  if constexpr (KIND != 0) return (int)(as_const(a.pos64)[b] + 1);
-  return as_const(a.ctx_lens)[b];
+__device__ __forceinline__ int seq_n(ArgsPtr a, int b) {
+  if constexpr (KIND != 0) return (int)(as_const(a->pos64)[b] + 1);
+  return as_const(a->ctx_lens)[b];
 }
 
 template <int KIND>
-__device__ __forceinline__ int page_id(const DecodeArgs& a, int b, int lp) {
-  const int idx = a.table_wrap > 0 ? lp % a.table_wrap : lp;
+__device__ __forceinline__ int page_id(ArgsPtr a, int b, int lp) {
+  const int idx = a->table_wrap > 0 ? lp % a->table_wrap : lp;
   int v;
   if constexpr (KIND == 2) {
-    v = (int)as_const(a.rows64)[b] * a.table_wrap + idx;
+    v = (int)as_const(a->rows64)[b] * a->table_wrap + idx;
   } else {
     // a logical page past the row's width has no entry: its keys are absent
     // (reading on would return the next row's page ids)
-    if ((unsigned)idx >= (unsigned)a.bt_width) return -1;
-    v = as_const(a.bt)[(int64_t)b * a.bt_stride + idx];
+    if ((unsigned)idx >= (unsigned)a->bt_width) return -1;
+    v = as_const(a->bt)[(int64_t)b * a->bt_stride + idx];
   }
-  // one unsigned 32-bit compare: stays on the scalar unit (a 64-bit signed
-  // compare would borrow VGPRs that in-flight loads may still own)
-  return (unsigned)v < (unsigned)a.num_pages ? v : -1;
+  return (unsigned)v < (unsigned)a->num_pages ? v : -1;
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t page_rsrc(const __bf16* pool,
-                                                            int phys,
-                                                            int page_bytes) {
-  const char* base = reinterpret_cast<const char*>(pool) +
-                     (phys >= 0 ? (int64_t)phys * page_bytes : 0);
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), (short)0,
-                                           phys >= 0 ? page_bytes : 0,
-                                           0x00020000);
-}
-
-// One 32-token step of the flattened page stream (wave-uniform).
+// One 32-token step of the flattened page stream (wave-uniform; small, since
+// three of them are held in scalar registers).
 struct Step {
   int b;       // sequence (-1: past the end of this work-group's range)
   int n;       // its context length
-  int s0, s1;  // its first and one-past-last unit in the page stream
   int pg;      // first logical page
-  int phys0, phys1;
-  bool first;  // first step of this piece: the query rows come with it
-  bool last;   // last step of this piece of sequence b
+  int flags;
+};
+enum : int {
+  kFirst = 1,   // first step of this piece: the query rows come with it
+  kLast = 2,    // last step of this piece of sequence b
+  kFull = 4,    // both pages present and all 32 tokens visible
+  kPage0 = 8,   // the pages are there
+  kPage1 = 16,
+  kWhole = 32,  // the piece is the whole sequence
 };
 
-template <bool REL>
-struct StepBuf {
-  u32x4 q[4];     // query fragments (first step of a piece only)
-  u32x4 k[2][4];  // [tile][load]: tokens 16 t + 4 i + (lane >> 4)
-  u32x4 v[2][4];
-  // raw bf16 bias bits of this lane's 8 scores, [4t + i] for token
-  // 16t + 4g + i; converted only when used, so issuing never waits
-  uint32_t rel[REL ? 8 : 1];
-};
+// distance of the step's first token
+__device__ __forceinline__ int rel_dist(const Step& st) {
+  return st.n - 1 - st.pg * kPS;
+}
 
-// Issue the loads of one 32-token step: the query fragments (from an
-// empty resource, i.e. no memory traffic, unless the step starts a piece:
-// a piece's query then never has to be waited for apart from its step),
-// 16 K/V buffer loads and, with a relative bias, the 8 bias values this
-// lane's scores need.
-template <bool REL>
-__device__ __forceinline__ void issue_step(StepBuf<REL>& buf,
-                                           const DecodeArgs& a,
-                                           const Step& st, int lane_off,
-                                           int page_bytes, int hq, bool head_ok,
-                                           int g) {
-  {
-    const bool want = st.first && st.b >= 0;
-    const char* base = reinterpret_cast<const char*>(a.q) +
-                       (want ? (int64_t)st.b * a.HQ * kD * 2 : 0);
-    __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(base), (short)0, want ? a.HQ * kD * 2 : 0,
-        0x00020000);
+// The bias of tile t's four scores of a lane out of the three dwords it
+// fetched: rel[d - i] for i = 0..3, zero from d - i = E on (the band's end).
+__device__ __forceinline__ void bias_values(const DecodeArgs& a, const Step& st,
+                                            const uint32_t (&w)[3], int t,
+                                            int sh, int g, float (&v)[4]) {
+  const uint32_t z0 = __builtin_amdgcn_alignbyte(w[1], w[0], sh);
+  const uint32_t z1 = __builtin_amdgcn_alignbyte(w[2], w[1], sh);
+  const uint32_t b[4] = {z1 & 0xffff0000u, z1 << 16, z0 & 0xffff0000u,
+                         z0 << 16};
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-      buf.q[kk] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rq, head_ok ? (hq * kD + 32 * kk + 8 * g) * 2 : 0x7ffffff0,
-                     0, 0));
-  }
-  if constexpr (REL) {
-    // rel row of sequence b: [HQ, E] bf16; out-of-band distances (and
-    // padded heads) get an out-of-range offset, which reads as 0
-    const char* base = reinterpret_cast<const char*>(a.rel) +
-                       (st.b >= 0 ? (int64_t)st.b * a.HQ * a.rel_extent * 2 : 0);
-    __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(base), (short)0,
-        st.b >= 0 ? a.HQ * a.rel_extent * 2 : 0, 0x00020000);
+  for (int i = 0; i < 4; ++i) v[i] = __builtin_bit_cast(float, b[i]);
+  const int d0 = rel_dist(st) - 16 * t;   // of the tile's oldest token
+  if (d0 >= a.rel_extent) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int dist = (st.n - 1) - ((st.pg + t) * kPS + 4 * g + i);
-        const bool in = head_ok && dist >= 0 && dist < a.rel_extent;
-        const int off = in ? (hq * a.rel_extent + dist) * 2 : 0x7ffffff0;
-        buf.rel[4 * t + i] = __builtin_amdgcn_raw_buffer_load_b16(
-            rr, off, 0, 0);
-      }
-  }
-  // lane l of load i reads 16 bytes of token 4i + (l >> 4): each group of
-  // 16 lanes reads one token's 256-byte head slice, so consecutive lanes
-  // are contiguous and every instruction coalesces into 64-byte requests
-  const int tok_b = page_bytes / kPS;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int phys = t == 0 ? st.phys0 : st.phys1;
-    __amdgpu_buffer_rsrc_t rk = page_rsrc(a.kpool, phys, page_bytes);
-    __amdgpu_buffer_rsrc_t rv = page_rsrc(a.vpool, phys, page_bytes);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      buf.k[t][i] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rk, lane_off + 4 * i * tok_b, 0, kStreamLoad));
-      buf.v[t][i] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rv, lane_off + 4 * i * tok_b, 0, kStreamLoad));
-    }
+    for (int i = 0; i < 4; ++i)
+      v[i] = d0 - 4 * g - i < a.rel_extent ? v[i] : 0.0f;
   }
 }
 
-// DEPTH: steps whose loads are in flight or being consumed; DEPTH - 1 steps
-// (16 KB each per wave) stream in while one is computed. One work-group per
-// CU (one wave per SIMD, the whole register file per wave).
-template <int REP, bool REL, int DEPTH, int KIND>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+// One work-group per CU by its LDS, one wave per SIMD. 256 registers: O^T then
+// stays in vector registers (given the whole register file the compiler kept
+// it in the accumulator half and moved all 32 values back and forth each step).
+template <int REP, bool REL, int KIND>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void decode_kernel(DecodeArgs a) {
   extern __shared__ __align__(16) char smem[];
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nw = blockDim.x >> 6;
   const int r = lane & 15;  // MFMA row / column index
   const int g = lane >> 4;  // MFMA k-group
   const int wg = blockIdx.x;
   const int G = gridDim.x;
   const int kvh = blockIdx.y * nw + w;
-  // the prefix table is only read before the walk; the per-wave K / V
-  // tiles then reuse the same LDS (a barrier separates the two uses)
+  // the tables of the batch (prefix of visible pages, lengths) are only read
+  // before the walk; the per-wave K / V tiles then reuse the same LDS (a
+  // barrier separates the two uses). The range's page ids follow both.
   int* pref = reinterpret_cast<int*>(smem);  // [B + 1]
   int* wsum = pref + a.B + 1;                // [4]
+  int* nlen = wsum + 4;                      // [B]
+  int* ids = reinterpret_cast<int*>(smem + a.ids_off);   // [ids_kept + 2]
 
   // ---- 1. prefix sums of visible pages: pref[b] = first unit of seq b ----
   {
     int carry = 0;
     for (int b0 = 0; b0 < a.B; b0 += blockDim.x) {
       const int b = b0 + threadIdx.x;
-      const int v = b < a.B ? vis_pages(seq_n<KIND>(a, b), a.window) : 0;
+      const int nb = b < a.B ? seq_n<KIND>(kernel_args(false), b) : 0;
+      const int v = vis_pages(nb, a.window);
+      if (b < a.B) nlen[b] = nb;
       // inclusive scan over the wave by DPP (VALU, no LDS round trips):
       // within each 16-lane row by shifts of 1, 2, 4, 8, then row 0's
       // total into row 1 and row 2's into row 3, then rows 0-1's total into
@@ -333,79 +300,224 @@ void decode_kernel(DecodeArgs a) {
   }
   if (u0 >= u1) return;
 
+  constexpr int kStageB = stage_bytes(REL);
   // ---- 3. the step stream of [u0, u1) -----------------------------------
-  // Everything about the step stream is wave-uniform and lives in SGPRs:
-  // the LDS prefix table is read only here, by the start-up binary search;
-  // afterwards the running prefix advances from scalar loads of ctx_lens,
-  // so no per-step LDS read needs a VGPR that an in-flight load still owns.
-  int cb;  // first sequence with pref[cb + 1] > u0
-  {
+  // Everything about the step stream is wave-uniform and lives in SGPRs. The
+  // page ids of the whole range are fetched here, one page per thread, into
+  // LDS: looked up step by step (a dependent scalar load or two per step,
+  // each waited for before the step's loads could go out) they cost every
+  // step several hundred cycles. The walk reads them one step ahead. In a
+  // range of more than kIds pages (a caller's own small grid, or contexts
+  // adding up to millions of tokens) the later ones are looked up step by
+  // step. Lengths of later sequences come from scalar loads.
+  constexpr int kIds = ids_kept(REL);
+  auto seq_of = [&](int u) {   // first sequence with pref[b + 1] > u
     int lo = 0, hi = a.B - 1;
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
-      if (__builtin_amdgcn_readfirstlane(pref[mid + 1]) > u0) hi = mid;
-      else lo = mid + 1;
+      if (pref[mid + 1] > u) hi = mid; else lo = mid + 1;
     }
-    cb = __builtin_amdgcn_readfirstlane(lo);
+    return lo;
+  };
+  const int nids = min(u1 - u0, kIds);
+  for (int i = threadIdx.x; i < nids; i += blockDim.x) {
+    const int b = seq_of(u0 + i);
+    ids[i] = page_id<KIND>(kernel_args(false), b,
+                           vis_lo(nlen[b], a.window) / kPS +
+                               (u0 + i - pref[b]));
   }
+  int cb = __builtin_amdgcn_readfirstlane(seq_of(u0));
   int seq_start = __builtin_amdgcn_readfirstlane(pref[cb]);
-  int cur_n = seq_n<KIND>(a, cb);
+  int cur_n = __builtin_amdgcn_readfirstlane(nlen[cb]);
   int seq_end = seq_start + vis_pages(cur_n, a.window);
+  int pg_of = vis_lo(cur_n, a.window) / kPS - seq_start;   // page of unit u
   int cu = u0;
   int last_b = -1;  // sequence of the previous step handed out
-  auto next_step = [&](Step& st) {
-    if (cu >= u1) {
-      st.b = -1; st.n = 0; st.pg = 0; st.phys0 = -1; st.phys1 = -1;
-      st.s0 = 0; st.s1 = 0; st.first = false; st.last = false;
-      return;
+  __syncthreads();  // the ids are there; every wave is done with the tables
+  // LDS address of the next step's ids (a range's first step is at least one
+  // page; what lies past its last page is read and not used)
+  uint32_t ids_at =
+      (uint32_t)(uintptr_t)((__attribute__((address_space(3))) int*)ids);
+  const uint32_t ids_end = ids_at + 4 * kIds;
+  int id0 = (int)lds_ld32(ids_at), id1 = (int)lds_ld32(ids_at + 4);
+  // The next step, and the pages it reads (-1: none).
+  auto next_step = [&](Step& st, int& phys0, int& phys1)
+      __attribute__((always_inline)) {
+    st.b = -1;
+    st.n = st.pg = st.flags = 0;
+    phys0 = phys1 = -1;
+    if (cu >= u1) return;
+    if (seq_end <= cu) {   // the next sequence that has a page
+      const ArgsPtr ra = kernel_args(true);
+      do {
+        ++cb;
+        seq_start = seq_end;
+        cur_n = seq_n<KIND>(ra, cb);
+        seq_end = seq_start + vis_pages(cur_n, a.window);
+      } while (seq_end <= cu);
+      pg_of = vis_lo(cur_n, a.window) / kPS - seq_start;
     }
-    while (seq_end <= cu) {
-      ++cb;
-      seq_start = seq_end;
-      cur_n = seq_n<KIND>(a, cb);
-      seq_end = seq_start + vis_pages(cur_n, a.window);
-    }
-    const int piece_end = min(seq_end, u1);
-    const int cnt = min(2, piece_end - cu);
+    const int cnt = min(2, min(seq_end, u1) - cu);
     st.b = cb;
     st.n = cur_n;
-    st.s0 = seq_start;
-    st.s1 = seq_end;
-    st.pg = vis_lo(cur_n, a.window) / kPS + (cu - seq_start);
-    st.phys0 = page_id<KIND>(a, cb, st.pg);
-    st.phys1 = cnt > 1 ? page_id<KIND>(a, cb, st.pg + 1) : -1;
+    st.pg = cu + pg_of;
+    phys0 = __builtin_amdgcn_readfirstlane(id0);
+    phys1 = __builtin_amdgcn_readfirstlane(id1);
+    if (ids_at + 4 * cnt > ids_end) {
+      const ArgsPtr ra = kernel_args(true);
+      phys0 = page_id<KIND>(ra, cb, st.pg);
+      phys1 = cnt > 1 ? page_id<KIND>(ra, cb, st.pg + 1) : -1;
+    }
+    if (cnt < 2) phys1 = -1;
     cu += cnt;
-    st.last = cu == piece_end;
-    st.first = cb != last_b;
+    ids_at = min(ids_at + 4 * cnt, ids_end);
+    id0 = (int)lds_ld32(ids_at);
+    id1 = (int)lds_ld32(ids_at + 4);
+    // every token visible: not before the window, not past the end
+    const int past = st.n - (st.pg + 2) * kPS;
+    const bool full = (phys0 | phys1) >= 0 && past >= 0 &&
+                      (a.window <= 0 || past + 2 * kPS <= a.window);
+    st.flags = (cb != last_b ? kFirst : 0) |
+               (cu == min(seq_end, u1) ? kLast : 0) | (full ? kFull : 0) |
+               (phys0 >= 0 ? kPage0 : 0) | (phys1 >= 0 ? kPage1 : 0) |
+               (seq_start >= u0 && seq_end <= u1 ? kWhole : 0);
     last_b = cb;
   };
 
   const int row_elems = (REP > 0 ? a.HKV : a.HKV_stored) * kD;
-  const int page_bytes = kPS * row_elems * 2;
   const int kvs = REP > 0 ? kvh : kvh / a.kv_div;   // the stored KV head
-  // byte offset of (token lane >> 4, head kvs, dims 8 (lane & 15)..) in a
-  // page
-  const int lane_off = ((lane >> 4) * row_elems + kvs * kD + 8 * (lane & 15)) * 2;
-  // this wave's LDS tiles: 32 token rows of 256 B each for K, then for V.
-  // K row x keeps 16-byte chunk c at slot c ^ (x & 15), V row x keeps
-  // 32-byte unit u at slot u ^ (x & 7): conflict-free for the row writes,
-  // for the K fragment reads (16 rows, one chunk) and for the transposed V
-  // reads (8 rows, one unit, per 32 lanes).
-  // The four lane-dependent bases below (multiples of 256 plus a swizzled
-  // slot) give every access as base ^ (slot bits) + immediate.
-  const uint32_t kt_l = (uint32_t)(uintptr_t)(
-      (__attribute__((address_space(3))) char*)smem) + w * kWaveLds;
-  const uint32_t vt_l = kt_l + kTileB;
-  const int wtok = lane >> 4, wch = lane & 15;  // row / chunk of a write
-  // write of load i, tile t: row x = 16t + 4i + wtok
-  const uint32_t kw0 = kt_l + wtok * kRowB + 16 * (wch ^ wtok);
-  const uint32_t vw0 = vt_l + wtok * kRowB + 32 * ((wch >> 1) ^ wtok) + 16 * (wch & 1);
-  // K fragment (t, kk) of lane (r, g): row 16t + r, chunk 4kk + g
-  const uint32_t kr0 = kt_l + r * kRowB + 16 * (g ^ r);
+  const int row_bytes = row_elems * 2;
+  // Tiles in LDS: 32 token rows of 256 B each for K, then for V. K row x
+  // keeps 16-byte chunk c at slot c ^ (x & 15), V row x keeps 32-byte unit u
+  // at slot u ^ (x & 7): conflict-free for the K fragment reads (16 rows, one
+  // chunk) and for the transposed V reads (8 rows, one unit, per 32 lanes).
+  // They arrive by direct loads, 4 rows per instruction: lane l fills row
+  // l >> 4, physical slot l & 15, and fetches the chunk that belongs there
+  // (a group of 16 lanes reads one token's whole 256-byte head slice).
+  const int wtok = lane >> 4, wslot = lane & 15;
+  int koff[4], voff[4];   // byte offsets in a page of rows 4i + wtok, less
+                          // the 1024 i that the instruction's own offset adds
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int x = 4 * i + wtok;
+    const int base = x * row_bytes + kvs * kRowB - 1024 * i;
+    koff[i] = base + 16 * (wslot ^ x);
+    voff[i] = base + 32 * ((wslot >> 1) ^ (x & 7)) + 16 * (wslot & 1);
+  }
+  const uint32_t lds_w =
+      (uint32_t)(uintptr_t)((__attribute__((address_space(3))) char*)smem) +
+      w * wave_lds(REL);
+  const uint32_t lds_q = lds_w + 2 * kStageB;
+  // K fragment (t, kk) of lane (r, g): row 16t + r, chunk 4kk + g (queries
+  // alike: row = head)
+  const uint32_t kr0 = lds_w + r * kRowB + 16 * (g ^ r);
   // transposed V reads: rows 4g + (s >> 2) (+16), unit blk, dims 4 (s & 3)
-  const int s16 = lane & 15;
-  const int x0 = 4 * g + (s16 >> 2);
-  const uint32_t vr0 = vt_l + x0 * kRowB + 32 * (x0 & 7) + 8 * (s16 & 3);
+  const int x0 = 4 * g + (wslot >> 2);
+  const uint32_t vr0 = lds_w + kTileB + x0 * kRowB + 32 * (x0 & 7) +
+                       8 * (wslot & 3);
+
+  // ---- direct loads of one step --------------------------------------------
+  // Always kNK for K and the bias, then 8 for V, whatever the step holds, so
+  // that the waits below can count: rows of a page that hold no visible key
+  // (and missing pages, and steps past the range) are outside the resource,
+  // arrive as zeros and are not fetched, so nothing has to be zeroed before
+  // P.V. (A page of the walk holds a visible key; a step's second page never
+  // holds the first one.)
+  constexpr int kRepMax = REP > 0 ? REP : 16;
+  constexpr int kNB = (kRepMax + 3) / 4 + 1;   // bias window loads
+  constexpr int kNK = REL ? 8 + kNB : 8, kNS = kNK + 8;
+  auto page_dma = [&](const __bf16* pool, const Step& st, int phys0, int phys1,
+                      uint32_t dst, const int (&off)[4])
+      __attribute__((always_inline)) {
+    const int past = st.n - st.pg * kPS;   // tokens from the step's first on
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int phys = t == 0 ? phys0 : phys1;
+      const int r_lo = t == 0 && a.window > 0 ? max(0, past - a.window) : 0;
+      const int r_hi = min(kPS, past - kPS * t);
+      const uint64_t base = (uint64_t)(uint32_t)max(phys, 0) *
+                                (uint32_t)(kPS * row_bytes) +
+                            (uint32_t)(r_lo * row_bytes);
+      const i32x4 rs =
+          make_rsrc(reinterpret_cast<const char*>(pool) + base,
+                    phys >= 0 ? (uint32_t)((r_hi - r_lo) * row_bytes) : 0u);
+      if (t == 0 && r_lo > 0) {   // the window's first page
+        const int d = r_lo * row_bytes;
+        dma4_nt<false>(rs, dst, off[0] - d, off[1] + 1024 - d,
+                       off[2] + 2048 - d, off[3] + 3072 - d);
+      } else {
+        dma4_nt<true>(rs, dst + t * kPS * kRowB, off[0], off[1], off[2],
+                      off[3]);
+      }
+    }
+  };
+  // Bias: of each head's row, the 32 values the step's tokens take (distances
+  // D - 31 .. D, D that of the first token): 17 dwords from the one that holds
+  // rel[D - 31]. 16 lanes fetch a head's first 16, four heads per load, into
+  // 64 bytes per head; one more load takes the 17th dwords. Dwords before the
+  // sequence's rows read as zeros; what they, or another row's values, put
+  // into a score past the band or masked is dropped. A step wholly past the
+  // band fetches nothing.
+  // byte offset of the 16-lane group's head row; padded heads: past every
+  // resource, whatever the distance adds
+  auto rel_row = [&](int hr) {
+    return hr < rep ? (kvh * rep + hr) * a.rel_extent * 2 : 0x60000000;
+  };
+  // byte offset of the sequence's first bias value in its dword (0 or 2), and
+  // the offset of distance D - 31 of a row, from the dword that holds it
+  auto rel_mis = [&](const Step& st) {
+    return (int)(((uintptr_t)a.rel +
+                  (int64_t)max(st.b, 0) * a.HQ * a.rel_extent * 2) & 3);
+  };
+  auto issue_k = [&](const Step& st, int phys0, int phys1, int stage)
+      __attribute__((always_inline)) {
+    const uint32_t dst = lds_w + stage * kStageB;
+    page_dma(a.kpool, st, phys0, phys1, dst, koff);
+    if constexpr (REL) {
+      const char* row = reinterpret_cast<const char*>(a.rel) +
+                        (int64_t)max(st.b, 0) * a.HQ * a.rel_extent * 2;
+      const int mis = rel_mis(st);
+      const bool band = st.b >= 0 && rel_dist(st) - 31 < a.rel_extent;
+      const i32x4 rs = make_rsrc(
+          row - mis,
+          band ? (uint32_t)((a.HQ * a.rel_extent * 2 + mis + 3) & ~3) : 0u);
+      const int d = 2 * (rel_dist(st) - 31) + mis;
+#pragma unroll
+      for (int j = 0; j + 1 < kNB; ++j)
+        dma32(rs, dst + 2 * kTileB + 256 * j,
+              (uint32_t)(((rel_row(4 * j + wtok) + d) & ~3) + 4 * wslot));
+      dma32(rs, dst + 2 * kTileB + 256 * (kNB - 1),
+            (uint32_t)(((rel_row(lane) + d) & ~3) + 64));
+    }
+  };
+  auto issue_v = [&](const Step& st, int phys0, int phys1, int stage)
+      __attribute__((always_inline)) {
+    page_dma(a.vpool, st, phys0, phys1, lds_w + stage * kStageB + kTileB, voff);
+  };
+  // where lane (r, g) finds the dwords of its scores of tile t (tokens
+  // 16t + 4g + i, i = 0..3: values 28 - 16t - 4g .. 31 - 16t - 4g of the
+  // window, from its dword 14 - 8t - 2g on): two adjacent ones and a third,
+  // which for t = g = 0 is the row's 17th (padded heads read the last row)
+  const int rr = min(r, rep - 1);
+  const uint32_t bias0 = lds_w + 2 * kTileB + 64 * rr + 4 * (14 - 2 * g);
+  const uint32_t bias2 =
+      g == 0 ? lds_w + 2 * kTileB + 256 * (kNB - 1) + 4 * rr : bias0 + 8;
+  // the 16 query rows of a piece (padded heads: zeros)
+  auto issue_q = [&](int b) __attribute__((always_inline)) {
+    const i32x4 rs = make_rsrc(
+        a.q + ((int64_t)b * a.HQ + (int64_t)kvh * rep) * kD,
+        (uint32_t)(rep * kRowB));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int x = 4 * i + wtok;
+      dma(rs, lds_q + 1024 * i, x * kRowB + 16 * (wslot ^ x));
+    }
+  };
+  // this wave's LDS reads are complete: what they read may be overwritten
+  auto lds_done = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));   // lgkmcnt 0
+    asm volatile("" ::: "memory");
+  };
 
   // ---- per-piece state ----------------------------------------------------
   f32x4 o_acc[8];
@@ -413,102 +525,7 @@ void decode_kernel(DecodeArgs a) {
   for (int blk = 0; blk < 8; ++blk) o_acc[blk] = f32x4{0, 0, 0, 0};
   float m_run = -INFINITY;
   float l_part = 0.0f;
-  bf16x8 qf[4];
-
-  auto compute = [&](const StepBuf<REL>& buf, const Step& st) {
-    const int n = st.n;
-    const int lo = vis_lo(n, a.window);
-    if (st.first) {
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) qf[kk] = __builtin_bit_cast(bf16x8, buf.q[kk]);
-    }
-    // ---- stage K and V rows in LDS -----------------------------------------
-    // (V rows of invalid tokens are zeroed: masked probabilities are 0 and
-    // must not meet a NaN in P.V)
-    const int k0 = st.pg * kPS;
-    wave_lds_sync();  // the previous step's fragment reads are done
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const bool page_ok = (t == 0 ? st.phys0 : st.phys1) >= 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // row x = 16t + 4i + wtok: x & 15 = 4i ^ wtok, x & 7 = 4(i & 1) ^ wtok
-        const int kpos = k0 + 16 * t + 4 * i + wtok;
-        const bool vok = page_ok && kpos >= lo && kpos < n;
-        const uint32_t rowo = (16 * t + 4 * i) * kRowB;
-        lds_st128((kw0 ^ (64u * i)) + rowo, buf.k[t][i]);
-        lds_st128((vw0 ^ (128u * (i & 1))) + rowo,
-                  vok ? buf.v[t][i] : u32x4{0, 0, 0, 0});
-      }
-    }
-    wave_lds_sync();
-    // ---- S^T = K.Q^T for the two 16-token tiles -------------------------
-    f32x4 sc[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      sc[t] = f32x4{0, 0, 0, 0};
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
-        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            lds_ld128((kr0 ^ (64u * kk)) + 16 * t * kRowB), qf[kk], sc[t], 0,
-            0, 0);
-    }
-    // ---- mask, bias, running max ----------------------------------------
-    float x[2][4];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const bool page_ok = (t == 0 ? st.phys0 : st.phys1) >= 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kpos = (st.pg + t) * kPS + 4 * g + i;
-        const bool ok = page_ok && kpos >= lo && kpos < n;
-        float v = sc[t][i] * a.scale_log2;
-        if constexpr (REL) v += bf16_bits_to_f32(buf.rel[4 * t + i]) * kLog2e;
-        v = ok ? v : -INFINITY;
-        x[t][i] = v;
-        mx = fmaxf(mx, v);
-      }
-    }
-    mx = lane_pair(lane_pair(mx, 16, true), 32, true);
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-    const float alpha = fast_exp2(m_run - m_use);
-    m_run = m_new;
-    // ---- probabilities: fp32 sum, bf16 operand --------------------------
-    // B-operand element j = 4t + i  <->  token 16t + 4g + i
-    float psum = 0.0f;
-    float p[2][4];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        p[t][i] = fast_exp2(x[t][i] - m_use);
-        psum += p[t][i];
-      }
-    l_part = l_part * alpha + psum;
-    uint32_t pw[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      pw[j] = pack_bf16x2(f32_to_bf16_bits(p[j >> 1][2 * (j & 1)]),
-                          f32_to_bf16_bits(p[j >> 1][2 * (j & 1) + 1]));
-    const bf16x8 pf =
-        __builtin_bit_cast(bf16x8, u32x4{pw[0], pw[1], pw[2], pw[3]});
-    // ---- O^T = O^T * alpha + V^T.P^T ------------------------------------
-    // A operand (dims 16 blk + r, tokens 4g..4g+3 and 16+4g..16+4g+3) by two
-    // transposed reads: source lane s of each 16-lane group names token
-    // base + (s >> 2) and dims 16 blk + 4 (s & 3)..+3
-#pragma unroll
-    for (int blk = 0; blk < 8; ++blk) {
-      const uint32_t va = vr0 ^ (32u * blk);
-      const bf16x4 lo4 = lds_tr16(va);
-      const bf16x4 hi4 = lds_tr16(va + 16 * kRowB);
-      const bf16x8 vf = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
-      o_acc[blk] = o_acc[blk] * alpha;
-      o_acc[blk] =
-          __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o_acc[blk], 0, 0, 0);
-    }
-  };
+  bf16x8 qf[4];   // query fragments
 
   // End of a piece of sequence b: write the result (whole sequence) or a
   // normalised partial that decode_combine_kernel merges.
@@ -523,15 +540,22 @@ void decode_kernel(DecodeArgs a) {
     // stay 32-bit, and padded heads / the LSE of lanes g != 0 / a missing
     // LSE output get an out-of-range offset or an empty resource (dropped),
     // so there is no divergent branch and no 64-bit address to keep live.
-    const int s0 = st.s0, s1 = st.s1;
-    const int bad = 0x7ffffff0;
-    if (s0 >= u0 && s1 <= u1) {
+    // (The lane's offset is opaque to the compiler, which would otherwise
+    // keep every store's offset in a register across the walk.)
+    const ArgsPtr ra = kernel_args(true);
+    const int HQ = ra->HQ;
+    const int bad = 0x7ffff000;
+    int eo = head_ok ? hq * kD + 4 * g : bad / 4;   // element of blk 0
+    int lo4 = head_ok && g == 0 ? hq * 4 : bad;
+    asm volatile("" : "+v"(eo), "+v"(lo4));
+    if (st.flags & kWhole) {
       const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-          reinterpret_cast<char*>(a.out + (int64_t)b * a.HQ * kD), (short)0,
-          a.HQ * kD * 2, 0x00020000);
+          reinterpret_cast<char*>(ra->out + (int64_t)b * HQ * kD), (short)0,
+          HQ * kD * 2, 0x00020000);
+      float* const lse = ra->lse;
       const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc(
-          reinterpret_cast<char*>(a.lse ? a.lse + (int64_t)b * a.HQ : nullptr),
-          (short)0, a.lse ? a.HQ * 4 : 0, 0x00020000);
+          reinterpret_cast<char*>(lse ? lse + (int64_t)b * HQ : nullptr),
+          (short)0, lse ? HQ * 4 : 0, 0x00020000);
 #pragma unroll
       for (int blk = 0; blk < 8; ++blk) {
         const uint32_t w0 =
@@ -541,30 +565,29 @@ void decode_kernel(DecodeArgs a) {
             pack_bf16x2(f32_to_bf16_bits(o_acc[blk][2] * inv),
                         f32_to_bf16_bits(o_acc[blk][3] * inv));
         __builtin_amdgcn_raw_buffer_store_b64(
-            u32x2{w0, w1}, ro,
-            head_ok ? (hq * kD + 16 * blk + 4 * g) * 2 : bad, 0, 0);
+            u32x2{w0, w1}, ro, eo * 2 + 32 * blk, 0, 0);
       }
       __builtin_amdgcn_raw_buffer_store_b32(
           __builtin_bit_cast(uint32_t, lse_nat), rl,
-          head_ok && g == 0 ? hq * 4 : bad, 0, 0);
+          lo4, 0, 0);
     } else {
       // one piece of a longer sequence: slot b + wg is unique because
       // work-groups and sequences are both laid out in order
-      const int64_t slot0 = (int64_t)(b + wg) * a.HQ;
+      const int64_t slot0 = (int64_t)(b + wg) * HQ;
       const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
-          reinterpret_cast<char*>(a.part_o + slot0 * kD), (short)0,
-          a.HQ * kD * 4, 0x00020000);
+          reinterpret_cast<char*>(ra->part_o + slot0 * kD), (short)0,
+          HQ * kD * 4, 0x00020000);
       const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc(
-          reinterpret_cast<char*>(a.part_lse + slot0), (short)0, a.HQ * 4,
+          reinterpret_cast<char*>(ra->part_lse + slot0), (short)0, HQ * 4,
           0x00020000);
 #pragma unroll
       for (int blk = 0; blk < 8; ++blk)
         __builtin_amdgcn_raw_buffer_store_b128(
             __builtin_bit_cast(u32x4, o_acc[blk] * inv), ro,
-            head_ok ? (hq * kD + 16 * blk + 4 * g) * 4 : bad, 0, 0);
+            eo * 4 + 64 * blk, 0, 0);
       __builtin_amdgcn_raw_buffer_store_b32(
           __builtin_bit_cast(uint32_t, lse_nat), rl,
-          head_ok && g == 0 ? hq * 4 : bad, 0, 0);
+          lo4, 0, 0);
     }
 #pragma unroll
     for (int blk = 0; blk < 8; ++blk) o_acc[blk] = f32x4{0, 0, 0, 0};
@@ -572,28 +595,174 @@ void decode_kernel(DecodeArgs a) {
     l_part = 0.0f;
   };
 
-  __syncthreads();  // every wave is done with the prefix table
-
-  // ---- 4. software-pipelined walk: next step's loads fly during math ----
-  // A ring of DEPTH step buffers: before step s is computed, the loads of
-  // step s + DEPTH - 1 go out into the buffer step s - 1 used. Steps past
-  // the range have no pages (zero-record resources: no memory traffic).
-  StepBuf<REL> buf[DEPTH];
-  Step stp[DEPTH];
+  // ---- 4. software-pipelined walk ------------------------------------------
+  // Step s sits in stage s & 1. Its fragments are read into registers first,
+  // each tile then makes room for step s + 2 at once, so two steps (32 KB per
+  // wave) are in flight while one is computed. With one wave per SIMD nothing
+  // hides a step's chain (fragment reads, score MFMAs, softmax, P.V MFMAs), so
+  // its length and its instruction count (4 cycles each) set how fast a
+  // compute unit streams: page rows do not pass through registers, V^T is
+  // read under the softmax, the next step's scalar work goes under the K
+  // reads, and steps whose 32 tokens are all visible skip the masks. Measured
+  // per step of 32 keys and 4 KV heads with its data in cache: 1.40 us for the
+  // form that loaded page rows into registers one step ahead, looked up page
+  // ids step by step and zeroed, masked and rescaled on every step (2.2 us
+  // with the bias, then 8 two-byte loads per lane); here 1.05 us (1.1 us), of
+  // which the chain is 0.66 us: the loads of one compute unit, 62 GB/s, now
+  // bound it. attn_swa at B = 4, 64Q/16KV (one ring per work-group): 37.3 ->
+  // 24.6 us; B = 96: 72.6 -> 65.3 us.
+  // Queries: those of the next step, if it starts a piece, go out at the top
+  // of this one.
+  Step cur, nx, nn;
+  int p0, p1;   // pages of the step whose loads go out
+  next_step(cur, p0, p1);
+  issue_q(cur.b);
+  issue_k(cur, p0, p1, 0);
+  issue_v(cur, p0, p1, 0);
+  next_step(nx, p0, p1);
+  issue_k(nx, p0, p1, 1);
+  issue_v(nx, p0, p1, 1);
+  auto read_q = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
 #pragma unroll
-  for (int k = 0; k < DEPTH - 1; ++k) {
-    next_step(stp[k]);
-    issue_step<REL>(buf[k], a, stp[k], lane_off, page_bytes, hq, head_ok, g);
-  }
+    for (int kk = 0; kk < 4; ++kk)
+      qf[kk] = lds_ld128((kr0 ^ (64u * kk)) + 2 * kStageB);
+    lds_done();
+  };
+  wait_vm<2 * kNS>();
+  read_q();
+  cur.flags &= ~kFirst;
   for (;;) {
 #pragma unroll
-    for (int k = 0; k < DEPTH; ++k) {
-      const int f = (k + DEPTH - 1) % DEPTH;
-      next_step(stp[f]);
-      issue_step<REL>(buf[f], a, stp[f], lane_off, page_bytes, hq, head_ok, g);
-      if (stp[k].b < 0) return;
-      compute(buf[k], stp[k]);
-      if (stp[k].last) finish_piece(stp[k]);
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t so = k * kStageB;
+      if (cur.flags & kFirst) {
+        wait_vm<kNS>();
+        read_q();
+      }
+      if (nx.flags & kFirst) issue_q(nx.b);
+      // ---- K fragments, bias dwords --------------------------------------------
+      wait_vm<8 + kNS>();   // after K(s), in flight: V(s) and step s + 1
+      asm volatile("" ::: "memory");
+      bf16x8 kf[2][4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          kf[t][kk] = lds_ld128((kr0 ^ (64u * kk)) + so + 16 * t * kRowB);
+      [[maybe_unused]] uint32_t bw[2][3];
+      if constexpr (REL) {
+        const u32x2 y0 = lds_ld64(bias0 + so), y1 = lds_ld64(bias0 + so - 32);
+        bw[0][0] = y0[0];
+        bw[0][1] = y0[1];
+        bw[0][2] = lds_ld32(bias2 + so);
+        bw[1][0] = y1[0];
+        bw[1][1] = y1[1];
+        bw[1][2] = lds_ld32(bias0 + so - 24);
+      }
+      next_step(nn, p0, p1);
+      lds_done();
+      // ---- S^T = K.Q^T for the two 16-token tiles -------------------------
+      f32x4 sc[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][kk], qf[kk],
+                                                          sc[t], 0, 0, 0);
+      issue_k(nn, p0, p1, k);
+      // ---- V^T fragments -------------------------------------------------------
+      // A operand (dims 16 blk + r, tokens 4g..4g+3 and 16+4g..16+4g+3) by two
+      // transposed reads: source lane s of each 16-lane group names token
+      // base + (s >> 2) and dims 16 blk + 4 (s & 3)..+3
+      wait_vm<kNS + kNK>();   // after V(s): step s + 1 and K(s + 2)
+      asm volatile("" ::: "memory");
+      bf16x8 vf[8];
+#pragma unroll
+      for (int blk = 0; blk < 8; ++blk) {
+        const uint32_t va = (vr0 ^ (32u * blk)) + so;
+        const bf16x4 lo4 = lds_tr16(va);
+        const bf16x4 hi4 = lds_tr16(va + 16 * kRowB);
+        vf[blk] = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+      __builtin_amdgcn_sched_barrier(0);   // (or the reads sink to their uses)
+      // ---- bias, mask, running max ----------------------------------------
+      float x[2][4];
+      float mx = -INFINITY;
+      [[maybe_unused]] int sh = 0;
+      if constexpr (REL)
+        sh = (rel_row(rr) + 2 * (rel_dist(cur) - 31) + rel_mis(cur)) & 2;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float bias[4];
+        if constexpr (REL) bias_values(a, cur, bw[t], t, sh, g, bias);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[t][i] = sc[t][i] * a.scale_log2;
+          if constexpr (REL) x[t][i] += bias[i] * kLog2e;
+        }
+      }
+      if (!(cur.flags & kFull)) {
+        const int lo = vis_lo(cur.n, a.window);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const bool page_ok = cur.flags & (t == 0 ? kPage0 : kPage1);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int kpos = (cur.pg + t) * kPS + 4 * g + i;
+            const bool ok = page_ok && kpos >= lo && kpos < cur.n;
+            x[t][i] = ok ? x[t][i] : -INFINITY;
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, x[t][i]);
+      mx = lane_pair(lane_pair(mx, 16, true), 32, true);
+      // O^T and l move to a new maximum only on the steps that have one (a
+      // reference that lags the maximum would skip more of them, but the
+      // largest probabilities are then no longer exact in bf16: 10% more error)
+      const bool move = mx > m_run;
+      if (__builtin_amdgcn_ballot_w64(move)) {
+        const float m_new = move ? mx : m_run;
+        const float alpha = move ? fast_exp2(m_run - m_new) : 1.0f;
+        m_run = m_new;
+        l_part *= alpha;
+#pragma unroll
+        for (int blk = 0; blk < 8; ++blk) o_acc[blk] = o_acc[blk] * alpha;
+      }
+      const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+      // ---- probabilities: fp32 sum, bf16 operand --------------------------
+      // B-operand element j = 4t + i  <->  token 16t + 4g + i
+      float p[2][4];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[t][i] = fast_exp2(x[t][i] - m_use);
+      l_part += ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) +
+                ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3]));
+      uint32_t pw[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        pw[j] = pack_bf16x2_rn(p[j >> 1][2 * (j & 1)],
+                               p[j >> 1][2 * (j & 1) + 1]);
+      const bf16x8 pf =
+          __builtin_bit_cast(bf16x8, u32x4{pw[0], pw[1], pw[2], pw[3]});
+      // ---- O^T += V^T.P^T ------------------------------------------------------
+      lds_done();
+#pragma unroll
+      for (int blk = 0; blk < 8; ++blk)
+        o_acc[blk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            vf[blk], pf, o_acc[blk], 0, 0, 0);
+      issue_v(nn, p0, p1, k);
+      if (cur.flags & kLast) finish_piece(cur);
+      cur = nx;
+      nx = nn;
+      if (cur.b < 0) {
+        wait_vm<0>();   // no direct load outlives the wave
+        return;
+      }
     }
   }
 }
@@ -678,10 +847,10 @@ template <int REP, int KIND>
 void launch_kind(const DecodeArgs& a, dim3 grid, int nw, size_t lds,
                  hipStream_t st) {
   if (a.rel)
-    hipLaunchKernelGGL((decode_kernel<REP, true, kDeep, KIND>), grid,
+    hipLaunchKernelGGL((decode_kernel<REP, true, KIND>), grid,
                        dim3(64 * nw), lds, st, a);
   else
-    hipLaunchKernelGGL((decode_kernel<REP, false, kDeep, KIND>), grid,
+    hipLaunchKernelGGL((decode_kernel<REP, false, KIND>), grid,
                        dim3(64 * nw), lds, st, a);
 }
 
@@ -865,9 +1034,10 @@ static int decode_impl(
   a.geo = (int*)((char*)workspace + off_geo);
 
   const int nw = waves_per_wg(a.HKV);
-  const size_t tab = ((size_t)B + 1 + 4) * sizeof(int);
-  const size_t tiles = (size_t)nw * kWaveLds;
-  const size_t lds = tab > tiles ? tab : tiles;
+  const size_t tab = ((2 * (size_t)B + 1 + 4) * sizeof(int) + 15) & ~(size_t)15;
+  const size_t tiles = (size_t)nw * wave_lds(rel != nullptr);
+  a.ids_off = (int)(tab > tiles ? tab : tiles);
+  const size_t lds = a.ids_off + (ids_kept(rel != nullptr) + 2) * sizeof(int);
   hipStream_t st = (hipStream_t)stream;
   switch (kv_div == 1 ? rep : 0) {
     case 1: launch<1>(a, G, nw, lds, st); break;

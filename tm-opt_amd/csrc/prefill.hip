@@ -64,54 +64,6 @@ constexpr int kRing = 4;                  // MFMA-phase fragment ring
 // checked below 2^31 - 16 on the host): the load returns zeros
 constexpr int kOob = 0x7ffffff0;
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-// raw buffer resource: base, byte range, dword 3 as for every buffer access
-// in this library
-// (all fields are wave-uniform; readfirstlane keeps them in scalar
-// registers, as the instruction needs, even where the compiler computed a
-// field with vector instructions)
-__device__ __forceinline__ i32x4 make_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t p = (uint64_t)(uintptr_t)base;
-  return i32x4{__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
-               __builtin_amdgcn_readfirstlane(
-                   (int)((uint32_t)(p >> 32) & 0xffffu)),
-               __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000};
-}
-
-// 16 bytes per lane from global memory straight into LDS: lane l of the
-// wave writes bytes lds + 16 l .. +15. Issued from inline assembly so that
-// the compiler does not wait for it at every barrier or before LDS reads it
-// cannot prove disjoint from it; the kernel waits for these loads itself
-// (wait_vm). The compiler's own waits for ordinary loads (the fused bias)
-// do not count these: they wait for every DMA issued between the load and
-// its use, so the tile loop issues no DMA in that stretch.
-__device__ __forceinline__ void dma(i32x4 rsrc, uint32_t lds, int voff) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-      :
-      : "s"(lds), "v"(voff), "s"(rsrc)
-      : "memory", "m0");
-}
-
-// 4 bytes per lane into LDS: lane l of the wave writes bytes lds + 4 l ..
-// +3 (the fused bias's window rows; the same rules as dma())
-__device__ __forceinline__ void dma32(i32x4 rsrc, uint32_t lds, uint32_t voff) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-      :
-      : "s"(lds), "v"(voff), "s"(rsrc)
-      : "memory", "m0");
-}
-
-// wait until at most N vector-memory loads of this wave are in flight
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) |
-                             (15 << 8));
-}
-
 struct PrefillArgs {
   const __bf16* q;
   int64_t q_st, q_sh;
