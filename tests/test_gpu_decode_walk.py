@@ -1,6 +1,6 @@
 """The decode walk's edges against the fp32 oracle: ranges of more page ids
 than the kernel keeps in LDS, rows of a window's first page that lie before
-the window, bias rows at every alignment."""
+the window, bias rows at every alignment, and the shapes of the merge."""
 from importlib import import_module
 
 import pytest
@@ -71,3 +71,23 @@ def test_bias_rows_at_every_alignment(tm, dev, hq, hkv, E):
     case = wl.make_decode("rel", 44, len(ctx), 0, 0, hq=hq, hkv=hkv, ctx=ctx)
     rel = torch.randn((len(ctx), hq, E), generator=g).bfloat16()
     _check(tm, dev, case, f"E={E} {hq}/{hkv}", rel, min_pages=2)
+
+
+@pytest.mark.parametrize("B,hq,hkv,pages", [
+    (1, 32, 4, 500), (1, 7, 1, 33), (2, 9, 3, 400), (5, 16, 2, 90),
+    (23, 32, 4, 40), (24, 32, 4, 40), (64, 8, 8, 12)])
+def test_merge_shapes(tm, dev, B, hq, hkv, pages):
+    """One piece per page (min_pages 1) over grids of 1 to 200 work-groups:
+    from a merge of 192 pieces by 32 groups per head to one of two pieces, an
+    odd number of heads per work-group, more groups than pieces, sequences
+    that need no merge beside ones that do."""
+    wl = import_module("tm-opt_amd.workloads")
+    g = torch.Generator().manual_seed(B)
+    ctx = torch.randint(1, 16 * pages, (B,), generator=g)
+    ctx[0] = 16 * pages
+    if B > 2:
+        ctx[1] = 3
+    case = wl.make_decode("merge", 45, B, 0, 0, hq=hq, hkv=hkv, ctx=ctx)
+    for wgs in (0, 7, 64, 200):
+        _check(tm, dev, case, f"merge B={B} wgs={wgs}", min_pages=1,
+               num_workgroups=wgs)

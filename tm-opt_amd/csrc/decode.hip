@@ -767,12 +767,17 @@ void decode_kernel(DecodeArgs a) {
   }
 }
 
-// Merge the pieces of every sequence that several work-groups shared:
-// grid (B, ceil(HQ / 8)), 8 heads x 32 lanes per work-group, 4 dims per
-// lane; pieces are merged in work-group order (deterministic, no atomics),
-// eight pieces' loads in flight at a time (one round for the pieces of most
-// sequences: the load latency, not the bytes, is what this kernel waits on).
-__global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a) {
+// Merge the pieces of every sequence that several work-groups shared, in a
+// fixed order (deterministic, no atomics): grid (B, ceil(HQ / H)), H heads per
+// work-group, S groups of 32 lanes per head (4 dims per lane). Group s takes
+// pieces s, s + S, ..., eight pieces' loads in flight at a time; the S results
+// then merge through LDS in group order. The load latency, not the bytes, is
+// what this kernel waits on: S is chosen so that the pieces of an average
+// sequence take one round (one 50,000-token sequence cut into 185 pieces:
+// 19.3 us with S = 1, 24 rounds in a chain, 5.0 us with S = 32).
+template <int H, int S>
+__global__ __launch_bounds__(32 * H * S) void decode_combine_kernel(
+    DecodeArgs a) {
   const int b = blockIdx.x;
   const int C = as_const(a.geo)[0];
   const int s0 = as_const(a.geo)[1 + b];
@@ -781,45 +786,82 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a) {
   const int wfirst = s0 / C;
   const int np = (s1 - 1) / C - wfirst + 1;
   if (np <= 1) return;                   // one piece: written in place
-  const int h = blockIdx.y * 8 + (threadIdx.x >> 5);
-  if (h >= a.HQ) return;
+  const int grp = threadIdx.x >> 5;
+  const int sub = grp % S;
+  const int h = blockIdx.y * H + grp / S;
+  const bool hok = h < a.HQ;
   const int d0 = 4 * (threadIdx.x & 31);
-  const int64_t slot0 = (int64_t)(b + wfirst) * a.HQ + h;
+  const int64_t slot0 = (int64_t)(b + wfirst) * a.HQ + (hok ? h : 0);
   float m = -INFINITY, sum = 0.0f;
   f32x4 acc = f32x4{0, 0, 0, 0};
+  auto add = [&](float l, float w1, f32x4 o) {   // a piece (LSE l, weight w1)
+    const float m_new = fmaxf(m, l);
+    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+    const float keep = fast_exp2((m - m_use) * kLog2e);
+    const float w = fast_exp2((l - m_use) * kLog2e);
+    sum = sum * keep + w * w1;
+    acc = acc * keep + o * w;
+    m = m_new;
+  };
   constexpr int kBatch = 8;
-  for (int k = 0; k < np; k += kBatch) {
+  for (int k = sub; k < np; k += kBatch * S) {
     float l4[kBatch];
     f32x4 o4[kBatch];
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
-      const bool in = k + j < np;
-      const int64_t slot = slot0 + (int64_t)(in ? k + j : 0) * a.HQ;
+      const bool in = k + j * S < np;
+      const int64_t slot = slot0 + (int64_t)(in ? k + j * S : 0) * a.HQ;
       l4[j] = in ? a.part_lse[slot] : -INFINITY;
       o4[j] = *reinterpret_cast<const f32x4*>(a.part_o + slot * kD + d0);
     }
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const float m_new = fmaxf(m, l4[j]);
-      const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-      const float keep = fast_exp2((m - m_use) * kLog2e);
-      const float w = fast_exp2((l4[j] - m_use) * kLog2e);
-      sum = sum * keep + w;
-      acc = acc * keep + o4[j] * w;
-      m = m_new;
+    for (int j = 0; j < kBatch; ++j) add(l4[j], 1.0f, o4[j]);
+  }
+  if constexpr (S > 1) {
+    // (m, sum, acc) of every group but the head's first, then merged by it
+    __shared__ float part[H * S][6][32];
+    const int l = threadIdx.x & 31;
+    if (sub > 0) {
+      part[grp][0][l] = m;
+      part[grp][1][l] = sum;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[grp][2 + i][l] = acc[i];
+    }
+    __syncthreads();
+    if (sub > 0) return;
+    const int n = min(np, S);
+    for (int j = 1; j < n; ++j) {
+      f32x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = part[grp + j][2 + i][l];
+      add(part[grp + j][0][l], part[grp + j][1][l], o);
     }
   }
+  if (!hok) return;
   const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
   __bf16* o = a.out + ((int64_t)b * a.HQ + h) * kD + d0;
   *reinterpret_cast<u32x2*>(o) =
-      u32x2{pack_bf16x2(f32_to_bf16_bits(acc[0] * inv),
-                        f32_to_bf16_bits(acc[1] * inv)),
-            pack_bf16x2(f32_to_bf16_bits(acc[2] * inv),
-                        f32_to_bf16_bits(acc[3] * inv))};
+      u32x2{pack_bf16x2_rn(acc[0] * inv, acc[1] * inv),
+            pack_bf16x2_rn(acc[2] * inv, acc[3] * inv)};
   if (a.lse && d0 == 0)
     a.lse[(int64_t)b * a.HQ + h] =
         sum > 0.0f ? (m == -INFINITY ? 0.0f : m) + fast_log2(sum) * kLn2
                    : -INFINITY;
+}
+
+// The merge's shape, from the number of pieces of an average sequence (at most
+// one more than its share of the grid's G ranges).
+void launch_combine(const DecodeArgs& a, int G, hipStream_t st) {
+  const int np = 1 + G / a.B;
+  if (np <= 8)
+    hipLaunchKernelGGL((decode_combine_kernel<8, 1>),
+                       dim3(a.B, (a.HQ + 7) / 8), dim3(256), 0, st, a);
+  else if (np <= 64)
+    hipLaunchKernelGGL((decode_combine_kernel<2, 8>),
+                       dim3(a.B, (a.HQ + 1) / 2), dim3(512), 0, st, a);
+  else
+    hipLaunchKernelGGL((decode_combine_kernel<1, 32>), dim3(a.B, a.HQ),
+                       dim3(1024), 0, st, a);
 }
 
 int waves_per_wg(int HKV) { return HKV % 4 == 0 ? 4 : (HKV % 2 == 0 ? 2 : 1); }
@@ -1049,8 +1091,7 @@ static int decode_impl(
   }
   int rc = check_launch("decode");
   if (rc || seqs_per_wg > 0) return rc;   // whole sequences: nothing to merge
-  hipLaunchKernelGGL(decode_combine_kernel, dim3(B, (HQ + 7) / 8), dim3(256),
-                     0, st, a);
+  launch_combine(a, G, st);
   return check_launch("decode_combine");
 }
 
