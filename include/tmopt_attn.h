@@ -380,6 +380,40 @@ int tmopt_attn_prefill_varlen(
     const int32_t* reject, tmopt_stream_t stream);
 
 /*
+ * The same with the keys of a query block split over several work-groups
+ * where the launch has fewer query blocks than the device compute units (a
+ * short chunk after a long cached context, a few short prompts): a second
+ * launch then merges the pieces, in a fixed order. workspace: device scratch
+ * of tmopt_attn_prefill_workspace_size bytes, 16-byte aligned, which needs no
+ * initialisation (TMOPT_EWORKSPACE if smaller; NULL, or a size of 0: one
+ * launch, as tmopt_attn_prefill_varlen).
+ */
+int tmopt_attn_prefill_varlen_split(
+    const void* q, int64_t q_stride_tok, int64_t q_stride_head, const void* k,
+    int64_t k_stride_run, int64_t k_stride_tok, int64_t k_stride_head,
+    int64_t k_stride_dim, const void* v, int64_t v_stride_run,
+    int64_t v_stride_tok, int64_t v_stride_head, int64_t v_stride_dim,
+    const int32_t* cu_seqlens_q,
+    const int32_t* prior_lens, int num_seqs, int max_seqlen_q,
+    const void* k_pool, const void* v_pool, const int32_t* block_table,
+    int64_t bt_stride, int table_wrap, int page_size, int64_t num_pages,
+    int HQ, int HKV, int D, int window, float scale, const void* rel,
+    int64_t rel_stride_tok, int64_t rel_stride_head, int rel_extent,
+    void* out, int64_t o_stride_tok, int64_t o_stride_head, float* lse,
+    const int32_t* reject, void* workspace, size_t workspace_bytes,
+    tmopt_stream_t stream);
+
+/*
+ * Bytes of workspace tmopt_attn_prefill_varlen_split needs for a launch shape
+ * on the current device; 0 where it does not split (bt_stride 0 without a
+ * block table). It does not depend on the lengths, which only the device
+ * knows: at most 2 x 129 KB per compute unit plus one round of query blocks.
+ */
+size_t tmopt_attn_prefill_workspace_size(int num_seqs, int max_seqlen_q,
+                                         int HQ, int HKV, int64_t bt_stride,
+                                         int table_wrap, int window);
+
+/*
  * The position contract of the reference's fused prefill
  * (engine/pyengine/kernels/attn_prefill.py:144-186: q_positions and
  * kv_positions [T] int64, the arange the engine builds, model.py:526-528),

@@ -77,6 +77,15 @@ SIGNATURES = {
         _c_i64, _c_i32, _c_i32, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
         _c_f32, _c_ptr, _c_i64, _c_i64, _c_i32,
         _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr]),
+    "tmopt_attn_prefill_varlen_split": (_c_i32, [
+        _c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64,
+        _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64,
+        _c_ptr, _c_ptr, _c_i32, _c_i32, _c_ptr, _c_ptr, _c_ptr,
+        _c_i64, _c_i32, _c_i32, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
+        _c_f32, _c_ptr, _c_i64, _c_i64, _c_i32,
+        _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
+    "tmopt_attn_prefill_workspace_size": (_c_size, [
+        _c_i32, _c_i32, _c_i32, _c_i32, _c_i64, _c_i32, _c_i32]),
     "tmopt_prefill_check_positions": (_c_i32, [
         _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr]),
 }

@@ -7,6 +7,8 @@ pointers, sizes and strides to libtmopt_attn.so on the current stream of the
 tensors' device. Nothing here computes attention: if the library is absent
 the call raises.
 """
+import functools
+
 import torch
 
 from . import _lib
@@ -340,6 +342,12 @@ def prefill_check_positions(q_positions, kv_positions, reject=None):
     return reject
 
 
+@functools.lru_cache(maxsize=1024)
+def _prefill_workspace_size(device, *shape):
+    """The library's answer for a launch shape, asked once per shape."""
+    return int(_lib.load().tmopt_attn_prefill_workspace_size(*shape))
+
+
 def prefill_varlen(q, k, v, cu_seqlens, scale, window=0, max_seqlen=None,
                    prior_lens=None, k_pool=None, v_pool=None,
                    block_table=None, table_wrap=0, rel=None, out=None,
@@ -370,6 +378,16 @@ def prefill_varlen(q, k, v, cu_seqlens, scale, window=0, max_seqlen=None,
     input rejection without a host sync).
     Returns (out [total, HQ, D] bf16, lse [HQ, total] fp32 or None).
     Reference: engine/pyengine/kernels/attn_prefill.py:71-194."""
+    return _prefill_varlen(q, k, v, cu_seqlens, scale, window, max_seqlen,
+                           prior_lens, k_pool, v_pool, block_table,
+                           table_wrap, rel, out, lse, return_lse, reject)
+
+
+def _prefill_varlen(q, k, v, cu_seqlens, scale, window, max_seqlen,
+                    prior_lens, k_pool, v_pool, block_table, table_wrap, rel,
+                    out, lse, return_lse, reject, split=True):
+    """prefill_varlen; split False: one launch, for a caller that fills the
+    rest of the device with other work."""
     total, HQ, D = q.shape
     _check_rows(q, "q")
     assert cu_seqlens.dtype == torch.int32 and cu_seqlens.dim() == 1
@@ -435,16 +453,24 @@ def prefill_varlen(q, k, v, cu_seqlens, scale, window=0, max_seqlen=None,
         out = torch.empty((total, HQ, D), dtype=torch.bfloat16, device=dev)
     if lse is None and return_lse:
         lse = torch.empty((HQ, total), dtype=torch.float32, device=dev)
-    _lib.call("tmopt_attn_prefill_varlen", _ptr(q), q.stride(0), q.stride(1),
+    # scratch for the pieces of a launch too small for the device (0 bytes
+    # for any other): the kernel splits its keys
+    bts = block_table.stride(0) if pooled else 0
+    n = _prefill_workspace_size(dev.index, S, int(max_seqlen), HQ, HKV, bts,
+                                int(table_wrap), int(window)) if split else 0
+    ws = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
+    _lib.call("tmopt_attn_prefill_varlen_split", _ptr(q), q.stride(0),
+              q.stride(1),
               _ptr(k) if own else None, *ks,
               _ptr(v) if own else None, *vs, _ptr(cu_seqlens),
               _ptr(prior_lens), S, int(max_seqlen),
               _ptr(k_pool) if pooled else None,
               _ptr(v_pool) if pooled else None, _ptr(block_table),
-              block_table.stride(0) if pooled else 0, int(table_wrap),
+              bts, int(table_wrap),
               page_size, P, HQ, HKV, D, int(window), float(scale), _ptr(rel),
               0 if rel is None else rel.stride(0),
               0 if rel is None else rel.stride(1),
               0 if rel is None else rel.shape[2], _ptr(out), out.stride(0),
-              out.stride(1), _ptr(lse), _ptr(reject), _stream(dev))
+              out.stride(1), _ptr(lse), _ptr(reject), _ptr(ws), n,
+              _stream(dev))
     return out, lse

@@ -1,13 +1,15 @@
 """In-tree build of libtmopt_attn.so for gfx950.
 
-One hipcc invocation compiles every HIP source of csrc/ into
-lib/libtmopt_attn.so. Packed FP32 instructions are disabled for all device
+The HIP sources of csrc/ are compiled side by side (one hipcc each) and
+linked into lib/libtmopt_attn.so. Packed FP32 instructions are disabled for all device
 code (-packed-fp32-ops); the host pass warns that it does not know the
 feature, which is harmless.
 """
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -15,10 +17,11 @@ LIB_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIB_DIR, "libtmopt_attn.so")
 ARCH = os.environ.get("TMOPT_ARCH", "gfx950")
 
-SOURCES = ["capi.hip", "kv_write.hip", "decode.hip", "prefill.hip"]
+SOURCES = ["capi.hip", "kv_write.hip", "decode.hip", "prefill.hip",
+           "prefill_split.hip"]
 
 FLAGS = [
-    f"--offload-arch={ARCH}", "-O3", "-fPIC", "-shared", "-std=c++17",
+    f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function",
 ]
@@ -30,13 +33,7 @@ def hipcc():
     return cand if os.path.exists(cand) else "hipcc"
 
 
-def build(verbose=False):
-    """Compile every source; raise CalledProcessError on failure."""
-    os.makedirs(LIB_DIR, exist_ok=True)
-    srcs = [os.path.join(CSRC, s) for s in SOURCES
-            if os.path.exists(os.path.join(CSRC, s))]
-    tmp = LIB + ".tmp"
-    cmd = [hipcc()] + FLAGS + srcs + ["-o", tmp]
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -48,6 +45,21 @@ def build(verbose=False):
                                             err)
     if verbose and err.strip():
         sys.stderr.write(err + "\n")
+
+
+def build(verbose=False):
+    """Compile every source; raise CalledProcessError on failure."""
+    os.makedirs(LIB_DIR, exist_ok=True)
+    tmp = LIB + ".tmp"
+    with tempfile.TemporaryDirectory() as d:
+        objs = [os.path.join(d, os.path.splitext(s)[0] + ".o")
+                for s in SOURCES]
+        cmds = [[hipcc()] + FLAGS + ["-c", os.path.join(CSRC, s), "-o", o]
+                for s, o in zip(SOURCES, objs)]
+        with ThreadPoolExecutor(len(cmds)) as pool:
+            list(pool.map(lambda c: _run(c, verbose), cmds))
+        _run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC"] + objs +
+             ["-o", tmp], verbose)
     os.replace(tmp, LIB)
     return LIB
 
