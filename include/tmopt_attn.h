@@ -246,6 +246,23 @@ int tmopt_attn_decode_ring(const void* q, const void* k_pool,
                            tmopt_stream_t stream);
 
 /*
+ * Paged decode over attn_global's own arguments
+ * (engine/pyengine/kernels/attn_global.py:15-38): flat [B, Lg] int64
+ * per-token pool rows as model.py:938-945 builds them (a page's rows are
+ * consecutive, so row 16 i names page i; pages from ceil(Lg / 16) on are
+ * absent) and pos [B] int64 query positions, read in place. Otherwise as
+ * tmopt_attn_decode_paged without a window, with the same results.
+ */
+int tmopt_attn_decode_flat(const void* q, const void* k_pool,
+                           const void* v_pool, const int64_t* flat,
+                           int64_t Lg, const int64_t* pos, int B, int HQ,
+                           int HKV, int D, int page_size, int64_t num_pages,
+                           float scale, const void* rel, int rel_extent,
+                           int min_pages, int num_workgroups, void* out,
+                           float* lse, void* workspace,
+                           size_t workspace_bytes, tmopt_stream_t stream);
+
+/*
  * The int32 block table and lengths of attn_global's arguments
  * (engine/pyengine/kernels/attn_global.py:15-38): flat [B, Lg] int64
  * per-token pool rows as model.py:938-945 builds them (flat[b, j] =

@@ -91,3 +91,54 @@ def test_merge_shapes(tm, dev, B, hq, hkv, pages):
     for wgs in (0, 7, 64, 200):
         _check(tm, dev, case, f"merge B={B} wgs={wgs}", min_pages=1,
                num_workgroups=wgs)
+
+
+@pytest.mark.parametrize("HQ,HK,E", [(64, 8, 1024), (12, 4, 33), (4, 4, 64)])
+def test_flat_rows_in_place(tm, dev, HQ, HK, E):
+    """decode_flat against decode_paged over the table made of the same rows:
+    bitwise (same kernel, same split); Lg a multiple of 16 and not, positions
+    past Lg (their pages are absent), row ids outside the pool."""
+    g = torch.Generator().manual_seed(46)
+    pos = torch.tensor([0, 15, 16, 700, 40, 1535, 1600, 333])
+    B, P = pos.shape[0], 900
+    kp = torch.randn((P, 16, HK, 128), generator=g).bfloat16().to(dev)
+    vp = torch.randn((P, 16, HK, 128), generator=g).bfloat16().to(dev)
+    q = torch.randn((B, HQ, 128), generator=g).bfloat16().to(dev)
+    rel = torch.randn((B, HQ, E), generator=g).bfloat16().to(dev)
+    for Lg in (1536, 1500, 17):
+        npg = -(-Lg // 16)
+        table = torch.randperm(P, generator=g)[:B * npg].view(B, npg)
+        table[3, npg // 2] = P + 5
+        j = torch.arange(Lg)
+        flat = table[:, j // 16] * 16 + (j % 16)[None]
+        flat = flat.masked_fill(j[None] > pos[:, None], 0).contiguous().to(dev)
+        t, n = tm.decode_table_from_flat(flat, pos.to(dev))
+        for r in (rel, None):
+            want = tm.decode_paged(q, kp, vp, t, n, 1 / 128, rel=r)
+            got = tm.decode_flat(q, kp, vp, flat, pos.to(dev), 1 / 128,
+                                 rel=r, return_lse=True)
+            torch.cuda.synchronize()
+            assert torch.equal(got[0], want[0]), (Lg, r is None)
+            assert torch.equal(got[1], want[1]), (Lg, r is None)
+
+
+def test_flat_rows_beyond_the_kept_page_ids(tm, dev):
+    """One work-group over more than 1500 pages of flat rows: the later ids
+    are looked up on the way."""
+    g = torch.Generator().manual_seed(47)
+    pos = torch.tensor([25000, 600])
+    Lg, P = 25001, 3200
+    kp = torch.randn((P, 16, 1, 128), generator=g).bfloat16().to(dev)
+    vp = torch.randn((P, 16, 1, 128), generator=g).bfloat16().to(dev)
+    q = torch.randn((2, 4, 128), generator=g).bfloat16().to(dev)
+    rel = torch.randn((2, 4, 100), generator=g).bfloat16().to(dev)
+    table = torch.randperm(P, generator=g)[:2 * 1563].view(2, 1563)
+    j = torch.arange(Lg)
+    flat = (table[:, j // 16] * 16 + (j % 16)[None]).contiguous().to(dev)
+    t, n = tm.decode_table_from_flat(flat, pos.to(dev))
+    want = tm.decode_paged(q, kp, vp, t, n, 1 / 128, rel=rel,
+                           num_workgroups=1)
+    got = tm.decode_flat(q, kp, vp, flat, pos.to(dev), 1 / 128, rel=rel,
+                         num_workgroups=1, return_lse=True)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

@@ -20,6 +20,7 @@ importlib.import_module("tm-opt_amd").
 from . import _lib
 from ._lib import TmoptError, TmoptLibraryMissing, version
 from .attn import (HEAD_DIM, PAGE_SIZE, decode_default_workgroups,
+                   decode_flat,
                    decode_paged, decode_paged_noalloc, decode_ring,
                    decode_table_from_flat, decode_workspace,
                    decode_workspace_size, kv_append_rows,
@@ -31,7 +32,8 @@ from .compat import (attn_global, attn_prefill_chunk_global,
 
 __all__ = [
     "TmoptError", "TmoptLibraryMissing", "version", "HEAD_DIM", "PAGE_SIZE",
-    "decode_default_workgroups", "decode_paged", "decode_paged_noalloc",
+    "decode_default_workgroups", "decode_flat", "decode_paged",
+    "decode_paged_noalloc",
     "decode_ring", "decode_table_from_flat", "decode_workspace",
     "prefill_check_positions",
     "decode_workspace_size", "kv_append_rows", "kv_write_paged",

@@ -64,6 +64,10 @@ SIGNATURES = {
         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i32, _c_ptr, _c_i32, _c_i32,
         _c_i32, _c_i32, _c_i64, _c_i32, _c_f32, _c_ptr, _c_i32, _c_i32,
         _c_i32, _c_i32, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
+    "tmopt_attn_decode_flat": (_c_i32, [
+        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i32, _c_i32,
+        _c_i32, _c_i32, _c_i32, _c_i64, _c_f32, _c_ptr, _c_i32, _c_i32,
+        _c_i32, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "tmopt_decode_table_from_flat": (_c_i32, [
         _c_ptr, _c_i64, _c_ptr, _c_i32, _c_ptr, _c_i64, _c_ptr, _c_ptr]),
     "tmopt_attn_decode_paged_noalloc": (_c_i32, [

@@ -273,6 +273,45 @@ def decode_ring(q, pool_k, pool_v, slots, pos, scale, window, rel=None,
     return out, lse
 
 
+def decode_flat(q, k_pool, v_pool, flat, pos, scale, rel=None, min_pages=8,
+                num_workgroups=0, out=None, lse=None, workspace=None,
+                return_lse=False):
+    """Paged decode over the engine's per-token rows: flat [B, Lg] int64
+    (model.py:938-945: row 16 i of a sequence names its page i) and pos [B]
+    int64 query positions, read in place (no block table or lengths built
+    per call); k_pool/v_pool [num_pages, 16, HKV, D].
+    Returns (out [B, HQ, D] bf16, lse [B, HQ] fp32 or None).
+    Reference: engine/pyengine/kernels/attn_global.py:15-38."""
+    B, HQ, D = q.shape
+    assert q.dtype == torch.bfloat16 and q.is_contiguous()
+    assert k_pool.is_contiguous() and v_pool.is_contiguous()
+    assert k_pool.dtype == torch.bfloat16 and v_pool.dtype == torch.bfloat16
+    assert k_pool.shape == v_pool.shape and k_pool.dim() == 4
+    P, page_size, HKV, Dk = k_pool.shape
+    assert Dk == D and HQ % HKV == 0, (k_pool.shape, q.shape)
+    assert flat.dtype == torch.int64 and flat.is_contiguous()
+    assert flat.dim() == 2 and flat.shape[0] == B
+    assert pos.dtype == torch.int64 and pos.shape == (B,)
+    assert pos.is_contiguous()
+    if rel is not None:
+        assert rel.dtype == torch.bfloat16 and rel.is_contiguous()
+        assert rel.shape[:2] == (B, HQ), (rel.shape, B, HQ)
+    dev = q.device
+    if out is None:
+        out = torch.empty_like(q)
+    if lse is None and return_lse:
+        lse = torch.empty((B, HQ), dtype=torch.float32, device=dev)
+    if workspace is None:
+        workspace = decode_workspace(B, HQ, HKV, dev, num_workgroups)
+    _lib.call("tmopt_attn_decode_flat", _ptr(q), _ptr(k_pool), _ptr(v_pool),
+              _ptr(flat), flat.shape[1], _ptr(pos), B, HQ, HKV, D, page_size,
+              P, float(scale), _ptr(rel),
+              0 if rel is None else rel.shape[2], int(min_pages),
+              int(num_workgroups), _ptr(out), _ptr(lse), _ptr(workspace),
+              workspace.numel() * workspace.element_size(), _stream(dev))
+    return out, lse
+
+
 def decode_table_from_flat(flat, pos, table=None, ctx_lens=None):
     """attn_global's per-token rows flat [B, Lg] int64 (model.py:938-945)
     and positions pos [B] int64 -> (block table [B, ceil(Lg/16)] int32 with

@@ -11,8 +11,8 @@ output layouts, and run the gfx950 kernels of this package:
     walked as a ring block table (table_wrap = W/16): position p lives in
     ring slot p % W, exactly RingKV's rule (kv.py:75-76, :99-100);
   * the global path's per-token flat rows `flat` [B, Lg] (model.py:938-945)
-    are turned back into a block table: rows of one page are consecutive,
-    so page i of row b is flat[b, 16 i] // 16;
+    are read in place: rows of one page are consecutive, so page i of row b
+    is flat[b, 16 i] // 16;
   * the padded [B, H, T, D] prefill batch becomes B runs of T tokens
     (cu_seqlens = 0, T, 2T, ...): queries as packed rows, K/V one run per
     batch row at the batch stride, token-major or channel-major (the sconv
@@ -74,9 +74,9 @@ def attn_global(q, pool_kp, pool_vp, flat, pos, rel, Lg):
     """Global decode attention over a page pool, in place (attn_global.py:15).
     q [B, HQ, D] bf16, pool_kp/pool_vp [(P+1), 16, HK, D] bf16, flat [B, Lg]
     i64 per-token rows (dead columns 0), pos [B] i64, rel [B, HQ, E] bf16.
-    Returns [B, HQ, D]. The block table is recovered from `flat` in one
-    launch (rows of one page are consecutive, so page i of row b is
-    flat[b, 16 i] // 16) together with the lengths pos + 1."""
+    Returns [B, HQ, D]. The kernel reads `flat` and `pos` in place: rows of
+    one page are consecutive, so page i of row b is flat[b, 16 i] // 16, and
+    the length is pos + 1."""
     B, HQ, D = q.shape
     assert q.is_contiguous() and rel.is_contiguous()
     assert pool_kp.is_contiguous() and pool_vp.is_contiguous()
@@ -84,9 +84,8 @@ def attn_global(q, pool_kp, pool_vp, flat, pos, rel, Lg):
     assert flat.dtype == torch.int64 and pos.dtype == torch.int64
     ps = pool_kp.shape[1]
     assert ps == PAGE
-    table, ctx = attn.decode_table_from_flat(flat, pos.contiguous())
-    out, _ = attn.decode_paged(q, pool_kp, pool_vp, table, ctx, 1.0 / D,
-                               window=0, rel=rel, return_lse=False)
+    out, _ = attn.decode_flat(q, pool_kp, pool_vp, flat, pos.contiguous(),
+                              1.0 / D, rel=rel)
     return out
 
 

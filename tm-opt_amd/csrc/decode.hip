@@ -90,10 +90,12 @@ struct DecodeArgs {
   int bt_width;      // entries a row may be read at: min(bt_stride, 2^31-1)
   int table_wrap;
   const int32_t* ctx_lens;
-  // the engine's own index tensors instead of a block table and lengths
-  // (tmopt_attn_decode_ring): kind 2 = ring slots [B] int64 (page
-  // slot * table_wrap + lp % table_wrap) and pos64 [B] int64 query
-  // positions (keys = pos + 1)
+  // the engine's own index tensors instead of a block table and lengths,
+  // with pos64 [B] int64 query positions (keys = pos + 1): kind 1
+  // (tmopt_attn_decode_flat) = per-token pool rows [B, bt_stride] int64 (page
+  // lp = row 16 lp / 16; bt_width counts its pages), kind 2
+  // (tmopt_attn_decode_ring) = ring slots [B] int64 (page slot * table_wrap +
+  // lp % table_wrap)
   int bt_kind;
   const int64_t* rows64;
   const int64_t* pos64;
@@ -160,7 +162,11 @@ __device__ __forceinline__ int page_id(ArgsPtr a, int b, int lp) {
     // a logical page past the row's width has no entry: its keys are absent
     // (reading on would return the next row's page ids)
     if ((unsigned)idx >= (unsigned)a->bt_width) return -1;
-    v = as_const(a->bt)[(int64_t)b * a->bt_stride + idx];
+    if constexpr (KIND == 1)
+      v = (int32_t)(as_const(a->rows64)[(int64_t)b * a->bt_stride +
+                                        (int64_t)kPS * idx] / kPS);
+    else
+      v = as_const(a->bt)[(int64_t)b * a->bt_stride + idx];
   }
   return (unsigned)v < (unsigned)a->num_pages ? v : -1;
 }
@@ -900,6 +906,7 @@ template <int REP>
 void launch(const DecodeArgs& a, int G, int nw, size_t lds, hipStream_t st) {
   const dim3 grid(G, a.HKV / nw);
   if (a.bt_kind == 2) launch_kind<REP, 2>(a, grid, nw, lds, st);
+  else if (a.bt_kind == 1) launch_kind<REP, 1>(a, grid, nw, lds, st);
   else launch_kind<REP, 0>(a, grid, nw, lds, st);
 }
 
@@ -971,11 +978,13 @@ extern "C" size_t tmopt_attn_decode_workspace_size(int B, int HQ, int HKV,
   return ws_layout(B, HQ, G, nullptr, nullptr);
 }
 
-// The decode launch behind both entry points: `kind` 0 = int32 block table
-// + int32 lengths (block_table, ctx_lens), 2 = ring slots + int64 positions
-// (rows64, pos64). (Per-token flat rows read in place, one page id per
-// 128 bytes, measured 17% slower than an int32 table at B = 64: every
-// page lookup missed the scalar cache ahead of the step's loads.)
+// The decode launch behind the entry points: `kind` 0 = int32 block table
+// + int32 lengths (block_table, ctx_lens), 1 = per-token flat rows + int64
+// positions (rows64, pos64), 2 = ring slots + int64 positions. (Flat rows,
+// one page id per 128 bytes, cost nothing over a table since a range's ids
+// are fetched at once: looked up step by step they measured 17% slower, and a
+// launch that makes a table of them first takes 4.8 us: 60.1 against 58.1 us
+// per call at 16 sequences of 1K-8K, 64Q/8KV.)
 static int decode_impl(
     int kind, const void* q, const void* k_pool, const void* v_pool,
     const int32_t* block_table, const int64_t* rows64, int64_t bt_stride,
@@ -1050,7 +1059,8 @@ static int decode_impl(
   a.vpool = (const __bf16*)v_pool;
   a.bt = block_table;
   a.bt_stride = bt_stride;
-  a.bt_width = bt_stride > 0x7fffffff ? 0x7fffffff : (int)bt_stride;
+  const int64_t width = kind == 1 ? (bt_stride + kPS - 1) / kPS : bt_stride;
+  a.bt_width = width > 0x7fffffff ? 0x7fffffff : (int)width;
   a.table_wrap = table_wrap;
   a.ctx_lens = ctx_lens;
   a.bt_kind = kind;
@@ -1125,6 +1135,20 @@ extern "C" int tmopt_attn_decode_ring(
                      window, scale, rel, rel_extent, min_pages,
                      num_workgroups, seqs_per_workgroup, out, lse, workspace,
                      workspace_bytes, stream);
+}
+
+extern "C" int tmopt_attn_decode_flat(
+    const void* q, const void* k_pool, const void* v_pool,
+    const int64_t* flat, int64_t Lg, const int64_t* pos, int B, int HQ,
+    int HKV, int D, int page_size, int64_t num_pages, float scale,
+    const void* rel, int rel_extent, int min_pages, int num_workgroups,
+    void* out, float* lse, void* workspace, size_t workspace_bytes,
+    tmopt_stream_t stream) {
+  clear_error();
+  return decode_impl(1, q, k_pool, v_pool, nullptr, flat, Lg, 0, nullptr, pos,
+                     B, HQ, HKV, D, page_size, num_pages, 0, scale, rel,
+                     rel_extent, min_pages, num_workgroups, 0, out, lse,
+                     workspace, workspace_bytes, stream);
 }
 
 extern "C" int tmopt_attn_decode_paged_noalloc(
