@@ -28,6 +28,7 @@ cache-populating paths take the rows' lengths from the host cache
 objects, as the reference's appends do (their small metadata tensors go
 through pinned memory, without a stream synchronisation).
 """
+import functools
 import os
 
 import torch
@@ -35,20 +36,36 @@ import torch
 from . import attn
 
 PAGE = attn.PAGE_SIZE
+# Fewest pages of a work-group's share in the decode adapters: one step of the
+# walk (a second one costs ~1 us, more than its part of the merge). Measured
+# at 8 / 4 / 2 pages, us per call: attn_swa, 2 rings, 64Q/16KV 14.0 / 12.3 /
+# 11.3; attn_global, 4 sequences up to 700, 64Q/8KV 15.1 / 13.2 / 12.1, 30 of
+# up to 200 16.6 / 13.9 / 13.1. A batch that gives every work-group more is
+# cut the same way for any of them.
+MIN_PAGES = 2
+
+
+@functools.lru_cache(maxsize=None)
+def _cus(device):
+    return torch.cuda.get_device_properties(device).multi_processor_count
 
 
 def _ring_grid(B, HKV, dev):
-    """Work split of a ring decode: k whole rings per work-group (k the
-    fewest that keep to one work-group per compute unit), so no row is
-    split between work-groups and the merge launch is skipped. Every row
-    holds at most W/16 pages, so full rings balance exactly. Measured at
-    B = 64, W = 512, 64Q/16KV: 52 us against 62 us with the default grid
-    (which splits rings and merges the pieces). Returns (work-groups, k)."""
+    """Work split of a ring decode (work-groups, whole rings per work-group;
+    0, 0: the default grid, which splits rows and merges the pieces). k whole
+    rings per work-group, k the fewest that keep to one work-group per
+    compute unit, need no merge launch and balance when the rings are full,
+    but stream fast only on enough compute units: the line is 0.6 of them.
+    Measured at W = 512, full rings, 64Q/16KV (whole rings / default grid,
+    us): B = 4 24.6 / 12.3, 32 (128 work-groups) 29.4 / 28.9, 40 (160) 32.9 /
+    34.9, 64 (256) 47.1 / 50.3, 72 (144 of two rings) 57.7 / 55.3, 80 (160)
+    58.0 / 60.4, 96 (192) 66.3 / 70.1; 32Q/4KV, B = 64 (64) 29.1 / 21.7."""
     groups = max(1, HKV // 4)
-    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    cus = _cus(dev.index)
     per_group = max(1, cus // groups)
     k = -(-B // per_group)
-    return -(-B // k), k
+    wgs = -(-B // k)
+    return (wgs, k) if 5 * wgs * groups >= 3 * cus else (0, 0)
 
 
 def attn_swa(q, pool_k, pool_v, slots, pos, rel):
@@ -66,7 +83,8 @@ def attn_swa(q, pool_k, pool_v, slots, pos, rel):
     wgs, k = _ring_grid(B, HK, q.device)
     out, _ = attn.decode_ring(q, pool_k, pool_v, slots.contiguous(),
                               pos.contiguous(), 1.0 / D, W, rel=rel,
-                              num_workgroups=wgs, seqs_per_workgroup=k)
+                              min_pages=MIN_PAGES, num_workgroups=wgs,
+                              seqs_per_workgroup=k)
     return out
 
 
@@ -85,7 +103,7 @@ def attn_global(q, pool_kp, pool_vp, flat, pos, rel, Lg):
     ps = pool_kp.shape[1]
     assert ps == PAGE
     out, _ = attn.decode_flat(q, pool_kp, pool_vp, flat, pos.contiguous(),
-                              1.0 / D, rel=rel)
+                              1.0 / D, rel=rel, min_pages=MIN_PAGES)
     return out
 
 
