@@ -144,6 +144,36 @@ int tmopt_kv_append_rows(const void* k, const void* v, int64_t k_stride_row,
                          void* k_pool, void* v_pool, int64_t num_pages,
                          tmopt_stream_t stream);
 
+/*
+ * K and V whose tokens are contiguous and whose head_dim is strided (the
+ * sconv output), laid out token-major: element (b, h, d, t) of k at
+ * b * k_stride_row + h * k_stride_head + d * k_stride_dim + t goes to
+ * k_out[((b * T + t) * HKV + h) * D + d] (likewise v), bit-exact, in one
+ * launch. For rows that the prefill and the KV write do not take in place
+ * (a token count that is not a multiple of 8). D == 128; k_out, v_out 16-byte
+ * aligned.
+ */
+int tmopt_pack_rows(const void* k, int64_t k_stride_row, int64_t k_stride_head,
+                    int64_t k_stride_dim, const void* v, int64_t v_stride_row,
+                    int64_t v_stride_head, int64_t v_stride_dim, int B, int T,
+                    int HKV, int D, void* k_out, void* v_out,
+                    tmopt_stream_t stream);
+
+/*
+ * The index tensors of a chunked prefill over the engine's storage
+ * (engine/pyengine/kv.py:215-268), in one launch: block_table
+ * [n_slots, width] int32 = table_dev[slots[b]] (GlobalPool's page table, table_rows rows of
+ * int64 at stride table_stride; NULL: slots[b] * width + i, a SwaPool ring of
+ * width pages), start_pos[b] = prior[b] for the n_prior runs and, if cu_seqlens is not NULL,
+ * cu_seqlens = {0, total}. A negative slot counts from the last row, as
+ * torch's indexing does; a slot outside the table names no page (-1).
+ */
+int tmopt_chunk_tables(const int64_t* table_dev, int64_t table_stride,
+                       int64_t table_rows, const int64_t* slots,
+                       int n_slots, const int64_t* prior, int n_prior,
+                       int width, int32_t* block_table, int32_t* start_pos,
+                       int32_t* cu_seqlens, int total, tmopt_stream_t stream);
+
 /* ------------------------------------------------------------------------ */
 /* Paged decode attention (split-KV + LSE combine)                          */
 /* ------------------------------------------------------------------------ */

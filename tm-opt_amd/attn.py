@@ -141,6 +141,40 @@ def kv_append_rows(k, v, lens, start_pos, block_table, k_pool, v_pool,
               _ptr(k_pool), _ptr(v_pool), P, _stream(k.device))
 
 
+def _pack_rows(k, v):
+    """[B, T, HKV, D] views of K and V with contiguous tokens (the sconv
+    output) -> token-major copies, one launch (tmopt_pack_rows)."""
+    B, T, HKV, D = k.shape
+    ko = torch.empty((B, T, HKV, D), dtype=torch.bfloat16, device=k.device)
+    vo = torch.empty_like(ko)
+    _lib.call("tmopt_pack_rows", _ptr(k), k.stride(0), k.stride(2),
+              k.stride(3), _ptr(v), v.stride(0), v.stride(2), v.stride(3), B,
+              T, HKV, D, _ptr(ko), _ptr(vo), _stream(k.device))
+    return ko, vo
+
+
+def _chunk_tables(slots, prior, width, table_dev=None, total=None):
+    """A chunk batch's block table [slots, width], start positions (prior)
+    and (with total) run bounds [2], all int32, in one launch
+    (tmopt_chunk_tables): rows `slots` of table_dev, or the rings `slots` of
+    width pages."""
+    assert slots.dim() == 1 and prior.dim() == 1
+    assert slots.device == prior.device
+    assert table_dev is None or table_dev.device == slots.device
+    slots, prior = slots.contiguous(), prior.contiguous()
+    B, S = slots.shape[0], prior.shape[0]
+    n = B * width
+    buf = torch.empty(n + S + 2, dtype=torch.int32, device=slots.device)
+    table, start, cu = buf[:n].view(B, width), buf[n:n + S], buf[n + S:]
+    _lib.call("tmopt_chunk_tables", _ptr(table_dev),
+              0 if table_dev is None else table_dev.stride(0),
+              0 if table_dev is None else table_dev.shape[0], _ptr(slots), B,
+              _ptr(prior), S, width, _ptr(table), _ptr(start),
+              None if total is None else _ptr(cu), total or 0,
+              _stream(slots.device))
+    return table, start, cu
+
+
 # --------------------------------------------------------------------------
 # Paged decode
 # --------------------------------------------------------------------------

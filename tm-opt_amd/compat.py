@@ -117,14 +117,12 @@ def _packed(x, B, T, H, D):
     return xt.as_strided((B * T, H, D), (xt.stride(1), xt.stride(2), 1))
 
 
-def _kv_rows(x):
-    """[B, HK, T, D] K or V (any strides) -> a [B, T, HK, D] view that the
-    prefill and the KV write both read in place: token-major rows (head_dim
-    contiguous) or channel-major ones (tokens contiguous, head_dim strided:
-    the sconv output, experiments/DEADENDS.md:631-645), with 16-byte
-    aligned rows, dim rows and heads. Anything else (e.g. channel-major with
-    T % 8 != 0) becomes a token-major copy, so a caller can rely on both
-    kernels accepting the result before it changes any cache."""
+def _in_place(x):
+    """[B, HK, T, D] K or V (any strides) -> its [B, T, HK, D] view, and
+    whether the prefill and the KV write both read that in place: token-major
+    rows (head_dim contiguous) or channel-major ones (tokens contiguous,
+    head_dim strided: the sconv output, experiments/DEADENDS.md:631-645), with
+    16-byte aligned rows, dim rows and heads."""
     xt = x.transpose(1, 2)                       # [B, T, HK, D]
     B, T, _, D = xt.shape
     if B == 1 and xt.stride(0) % 8 != 0:
@@ -136,9 +134,30 @@ def _kv_rows(x):
     token_major = st[3] == 1 and st[1] % 8 == 0
     channel_major = (st[1] == 1 and D == attn.HEAD_DIM and st[3] % 8 == 0 and
                      st[3] >= T)
-    if aligned and (token_major or channel_major):
-        return xt
-    return xt.contiguous()
+    return xt, aligned and (token_major or channel_major)
+
+
+def _kv_rows(x):
+    """[B, HK, T, D] K or V (any strides) -> a [B, T, HK, D] view that the
+    prefill and the KV write both read in place (see _in_place). Anything else
+    (e.g. channel-major with T % 8 != 0) becomes a token-major copy, so a
+    caller can rely on both kernels accepting the result before it changes any
+    cache."""
+    xt, ok = _in_place(x)
+    return xt if ok else xt.contiguous()
+
+
+def _kv_pair(k, v):
+    """_kv_rows of K and V. Channel-major rows that neither kernel reads in
+    place (the sconv output at T % 8 != 0) are laid out in one launch."""
+    (kt, k_ok), (vt, v_ok) = _in_place(k), _in_place(v)
+    if (not k_ok and not v_ok and k.is_cuda and kt.stride(1) == 1 and
+            vt.stride(1) == 1 and kt.shape[3] == attn.HEAD_DIM and
+            kt.dtype == vt.dtype == torch.bfloat16 and
+            kt.shape == vt.shape and kt.device == vt.device and 0 < kt.shape[0] <= 65535 and
+            0 < kt.shape[2] <= 32767):
+        return attn._pack_rows(kt, vt)
+    return (kt if k_ok else kt.contiguous(), vt if v_ok else vt.contiguous())
 
 
 def _to_device(rows, dev):
@@ -333,7 +352,7 @@ def attn_prefill_fused(q, k, v, rel, q_positions, kv_positions, window,
     out = torch.empty((B, T, H, D), dtype=q.dtype, device=dev)
     cu = _uniform_cu(B, T, dev)
     w = 0 if window is None else int(window)
-    kr, vr = _kv_rows(k), _kv_rows(v)            # [B, T, HK, D]
+    kr, vr = _kv_pair(k, v)                      # [B, T, HK, D]
     if caches is not None:
         assert len(caches) == B
         assert all(int(c.n) == 0 for c in caches), \
@@ -360,20 +379,17 @@ def attn_prefill_fused(q, k, v, rel, q_positions, kv_positions, window,
 # after the attention, which a ring requires (it overwrites positions the
 # chunk's first queries still see).
 
-def _chunk_cu(q, cu_seqlens, max_seqlen):
-    """(cu_seqlens, max_seqlen) of a chunk batch: one sequence of
-    q.shape[0] tokens when cu_seqlens is None (no device read); otherwise
-    max_seqlen as given, or read back once (a host synchronisation, which a
-    graph capture must avoid by passing it) for both launches."""
+def _chunk_max(q, cu_seqlens, max_seqlen):
+    """The longest chunk of a batch: q.shape[0] for one sequence (cu_seqlens
+    None), otherwise max_seqlen as given, or read back once (a host
+    synchronisation, which a graph capture must avoid by passing it) for both
+    launches."""
     if cu_seqlens is None:
-        cu = torch.full((2,), q.shape[0], dtype=torch.int32,
-                        device=q.device)
-        cu[0] = 0
-        return cu, q.shape[0]
+        return q.shape[0]
     assert cu_seqlens.dtype == torch.int32
     if max_seqlen is None:
         max_seqlen = int((cu_seqlens[1:] - cu_seqlens[:-1]).max())
-    return cu_seqlens, max_seqlen
+    return max_seqlen
 
 
 def attn_prefill_chunk_swa(q, k, v, rel, pool_k, pool_v, slots, prior,
@@ -396,13 +412,14 @@ def attn_prefill_chunk_swa(q, k, v, rel, pool_k, pool_v, slots, prior,
     assert slots.dtype == torch.int64 and prior.dtype == torch.int64
     if rel is not None:
         assert rel.shape == (total, H, W), (rel.shape, (total, H, W))
-    cu, max_seqlen = _chunk_cu(q, cu_seqlens, max_seqlen)
+    max_seqlen = _chunk_max(q, cu_seqlens, max_seqlen)
     per = W // PAGE
     kp = pool_k.view(S1 * per, PAGE, HK, D)
     vp = pool_v.view(S1 * per, PAGE, HK, D)
-    table = (slots[:, None] * per + torch.arange(
-        per, device=q.device, dtype=torch.int64)[None]).to(torch.int32)
-    start = prior.to(torch.int32)
+    table, start, cu = attn._chunk_tables(
+        slots, prior, per, total=total if cu_seqlens is None else None)
+    if cu_seqlens is not None:
+        cu = cu_seqlens
     out, _ = attn.prefill_varlen(q, k, v, cu, 1.0 / D, window=W,
                                  max_seqlen=max_seqlen, prior_lens=start,
                                  k_pool=kp, v_pool=vp, block_table=table,
@@ -433,9 +450,14 @@ def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
     assert slots.dtype == torch.int64 and prior.dtype == torch.int64
     if rel is not None:
         assert rel.shape[:2] == (total, H)
-    cu, max_seqlen = _chunk_cu(q, cu_seqlens, max_seqlen)
-    table = table_dev[slots].to(torch.int32)
-    start = prior.to(torch.int32)
+    max_seqlen = _chunk_max(q, cu_seqlens, max_seqlen)
+    if table_dev.stride(1) != 1 or table_dev.stride(0) < table_dev.shape[1]:
+        table_dev = table_dev.contiguous()
+    table, start, cu = attn._chunk_tables(
+        slots.to(table_dev.device), prior, table_dev.shape[1], table_dev,
+        total if cu_seqlens is None else None)
+    if cu_seqlens is not None:
+        cu = cu_seqlens
     out, _ = attn.prefill_varlen(q, k, v, cu, 1.0 / D, window=0,
                                  max_seqlen=max_seqlen, prior_lens=start,
                                  k_pool=pool_kp, v_pool=pool_vp,

@@ -260,6 +260,84 @@ __global__ __launch_bounds__(256) void kv_write_paged_cm_kernel(
   }
 }
 
+// ---- channel-major rows that neither reader takes in place ----------------
+// Rows of a token count that is not a multiple of 8 start at any even byte,
+// which no 16-byte load takes. K and V [B, HKV, D, T] (tokens contiguous, any
+// other strides) are then laid out token-major, [B, T, HKV, D], in one launch:
+// a work-group moves 64 tokens x 128 dims of one head of K or of V through
+// LDS, reading a dim's 64 tokens per wave (128 bytes, two per lane) and
+// writing whole 256-byte rows. LDS rows (one token) are 130 elements apart, so
+// the two-byte writes of a wave (64 tokens of one dim, 65 dwords apart) spread
+// over all banks. Two tensors of 777 tokens, 8 heads: 15.3 us for two strided
+// copies, PACKUS here.
+constexpr int kPackTok = 64;
+constexpr int kPackRow = 130;
+__global__ __launch_bounds__(256) void pack_rows_kernel(
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    int64_t k_sb, int64_t k_sh, int64_t k_sd, int64_t v_sb, int64_t v_sh,
+    int64_t v_sd, int T, int HKV, uint16_t* __restrict__ ko,
+    uint16_t* __restrict__ vo) {
+  __shared__ uint16_t tile[kPackTok * kPackRow];
+  const int h = blockIdx.y % HKV;
+  const bool is_v = (int)blockIdx.y >= HKV;
+  const int64_t b = blockIdx.z;
+  const int t0 = kPackTok * (int)blockIdx.x;
+  const uint16_t* src = is_v ? v + b * v_sb + h * v_sh : k + b * k_sb + h * k_sh;
+  const int64_t sd = is_v ? v_sd : k_sd;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int t = min(t0 + lane, T - 1);      // (tokens past the end: not stored)
+  uint16_t x[32];
+#pragma unroll
+  for (int j = 0; j < 32; ++j) x[j] = src[(int64_t)(32 * w + j) * sd + t];
+#pragma unroll
+  for (int j = 0; j < 32; ++j) tile[lane * kPackRow + 32 * w + j] = x[j];
+  __syncthreads();
+  // 64 lanes write one token's 128 dims, 4 bytes each
+  uint32_t* out = reinterpret_cast<uint32_t*>(is_v ? vo : ko);
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int tok = 16 * w + j;
+    const uint32_t y = *reinterpret_cast<const uint32_t*>(
+        &tile[tok * kPackRow + 2 * lane]);
+    if (t0 + tok < T)
+      out[((b * T + t0 + tok) * HKV + h) * (kCmD / 2) + lane] = y;
+  }
+}
+
+// ---- the chunk adapters' index tensors -------------------------------------
+// Block table, start positions and run bounds of a chunk batch from the
+// engine's own: table[b][i] = table_dev[slots[b]][i] (GlobalPool's device page
+// table, rows x width int64), or slots[b] * ring_pages + i without one (a ring
+// of ring_pages = width pages); start[b] = prior[b]; with `cu`, one run of
+// `total` rows. A slot counts from the end if negative, as torch's indexing
+// does; the entries of one outside the table are -1 (no page).
+__global__ __launch_bounds__(256) void chunk_tables_kernel(
+    const int64_t* __restrict__ table_dev, int64_t row_stride, int64_t rows,
+    const int64_t* __restrict__ slots, int n_slots,
+    const int64_t* __restrict__ prior, int n_prior, int width, int32_t* __restrict__ table, int32_t* __restrict__ start,
+    int32_t* __restrict__ cu, int total) {
+  const int b = blockIdx.y;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (b < n_slots && i < width) {
+    int64_t s = slots[b];
+    int32_t page;
+    if (table_dev != nullptr) {
+      if (s < 0) s += rows;
+      page = s >= 0 && s < rows ? (int32_t)table_dev[s * row_stride + i] : -1;
+    } else {
+      page = (int32_t)(s * width + i);
+    }
+    table[(int64_t)b * width + i] = page;
+  }
+  if (i == 0) {
+    if (b < n_prior) start[b] = (int32_t)prior[b];
+    if (cu != nullptr && b == 0) {
+      cu[0] = 0;
+      cu[1] = total;
+    }
+  }
+}
+
 int check_kv_common(const void* k, const void* v, int64_t k_st, int64_t k_sh,
                     int64_t v_st, int64_t v_sh, int HKV, int D,
                     const void* kp, const void* vp) {
@@ -455,4 +533,58 @@ extern "C" int tmopt_kv_append_rows(
                      k_stride_row, v_stride_row, start_pos, num_rows, max_len,
                      block_table, bt_stride, table_wrap, page_size, HKV, D,
                      k_pool, v_pool, num_pages, stream);
+}
+
+extern "C" int tmopt_pack_rows(const void* k, int64_t k_stride_row,
+                               int64_t k_stride_head, int64_t k_stride_dim,
+                               const void* v, int64_t v_stride_row,
+                               int64_t v_stride_head, int64_t v_stride_dim,
+                               int B, int T, int HKV, int D, void* k_out,
+                               void* v_out, tmopt_stream_t stream) {
+  clear_error();
+  if (B == 0 || T == 0) return TMOPT_OK;
+  TMOPT_REQUIRE(B > 0 && B <= 65535 && T > 0 && HKV > 0 && HKV <= 32767,
+                TMOPT_EINVAL, "pack_rows: B=%d T=%d HKV=%d", B, T, HKV);
+  TMOPT_REQUIRE(D == kCmD, TMOPT_EUNSUPPORTED, "pack_rows: D=%d (only %d)", D,
+                kCmD);
+  TMOPT_REQUIRE(k && v && k_out && v_out, TMOPT_EINVAL,
+                "pack_rows: null tensor pointer");
+  TMOPT_REQUIRE(((uintptr_t)k | (uintptr_t)v) % 2 == 0 &&
+                    ((uintptr_t)k_out | (uintptr_t)v_out) % 16 == 0,
+                TMOPT_EINVAL, "pack_rows: misaligned tensor");
+  hipLaunchKernelGGL(pack_rows_kernel,
+                     dim3((unsigned)((T + kPackTok - 1) / kPackTok), 2 * HKV, B),
+                     dim3(256), 0, (hipStream_t)stream, (const uint16_t*)k,
+                     (const uint16_t*)v, k_stride_row, k_stride_head,
+                     k_stride_dim, v_stride_row, v_stride_head, v_stride_dim,
+                     T, HKV, (uint16_t*)k_out, (uint16_t*)v_out);
+  return check_launch("pack_rows");
+}
+
+extern "C" int tmopt_chunk_tables(const int64_t* table_dev,
+                                  int64_t table_stride, int64_t table_rows,
+                                  const int64_t* slots, int n_slots,
+                                  const int64_t* prior, int n_prior,
+                                  int width, int32_t* block_table,
+                                  int32_t* start_pos, int32_t* cu_seqlens,
+                                  int total, tmopt_stream_t stream) {
+  clear_error();
+  if (n_slots == 0 && n_prior == 0) return TMOPT_OK;
+  TMOPT_REQUIRE(n_slots >= 0 && n_slots <= 65535 && n_prior >= 0 &&
+                    n_prior <= 65535 && width > 0,
+                TMOPT_EINVAL, "chunk_tables: slots=%d prior=%d width=%d",
+                n_slots, n_prior, width);
+  TMOPT_REQUIRE(slots && prior && block_table && start_pos, TMOPT_EINVAL,
+                "chunk_tables: null pointer");
+  TMOPT_REQUIRE(table_dev == nullptr ||
+                    (table_rows > 0 && table_stride >= width),
+                TMOPT_EINVAL, "chunk_tables: rows=%lld stride=%lld width=%d",
+                (long long)table_rows, (long long)table_stride, width);
+  hipLaunchKernelGGL(chunk_tables_kernel,
+                     dim3((unsigned)((width + 255) / 256),
+                          (unsigned)(n_slots > n_prior ? n_slots : n_prior)),
+                     dim3(256), 0, (hipStream_t)stream, table_dev,
+                     table_stride, table_rows, slots, n_slots, prior, n_prior,
+                     width, block_table, start_pos, cu_seqlens, total);
+  return check_launch("chunk_tables");
 }
