@@ -142,3 +142,25 @@ def test_flat_rows_beyond_the_kept_page_ids(tm, dev):
                          num_workgroups=1, return_lse=True)
     torch.cuda.synchronize()
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("B,pages", [(1, 500), (5, 90), (24, 40)])
+def test_merge_of_infinite_values(tm, dev, B, pages):
+    """An infinity in V is one in that dim's output of the heads that read
+    it, whatever the number of pieces the merge rounds up to, and no NaN."""
+    wl = import_module("tm-opt_amd.workloads")
+    case = wl.make_decode("inf", 48, B, 0, 0, hq=8, hkv=2,
+                          ctx=[16 * pages] * B)
+    for b in range(B):
+        case.v_pool[int(case.block_table[b, 0]), 5, 1, 3] = float("inf")
+    c = case.to(dev)
+    want = torch.zeros((B, 8, 128), dtype=torch.bool)
+    want[:, 4:, 3] = True
+    for wgs in (0, 7, 64):
+        out, _ = tm.decode_paged(c.q, c.k_pool, c.v_pool, c.block_table,
+                                 c.ctx_lens, 0.01, min_pages=1,
+                                 num_workgroups=wgs)
+        torch.cuda.synchronize()
+        out = out.cpu()
+        assert torch.equal(out.isinf(), want), wgs
+        assert not out.isnan().any(), wgs

@@ -136,3 +136,20 @@ def test_split_repeats_bitwise_and_matches_one_launch(tm, dev):
         finally:
             tm._lib.call = real
     assert e.value.status == tm._lib.TMOPT_EWORKSPACE
+
+
+@pytest.mark.parametrize("prior", [1500, 4000])
+def test_infinite_values(tm, dev, prior):
+    """An infinity in V that every query sees, in the last piece, is one in
+    each of their outputs of that dim and KV head, and no NaN anywhere."""
+    wl = import_module("tm-opt_amd.workloads")
+    a = _runs([40], [prior], 16, 2, 71, "paged", wl)
+    a["v_pool"][int(a["block_table"][0, prior // 16]), 0, 1, 3] = float("inf")
+    a["scale"] = 0.01            # no probability of that key rounds to zero
+    d = {k: v.to(dev) if torch.is_tensor(v) else v for k, v in a.items()}
+    out, _ = tm.prefill_varlen(**d)
+    torch.cuda.synchronize()
+    want = torch.zeros(out.shape, dtype=torch.bool)
+    want[:, 8:, 3] = True
+    out = out.cpu()
+    assert torch.equal(out.isinf(), want) and not out.isnan().any()

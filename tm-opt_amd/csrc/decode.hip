@@ -821,7 +821,8 @@ __global__ __launch_bounds__(32 * H * S) void decode_combine_kernel(
       o4[j] = *reinterpret_cast<const f32x4*>(a.part_o + slot * kD + d0);
     }
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) add(l4[j], 1.0f, o4[j]);
+    for (int j = 0; j < kBatch; ++j)     // (0 x infinity: weight 0 won't do)
+      add(l4[j], 1.0f, k + j * S < np ? o4[j] : f32x4{0, 0, 0, 0});
   }
   if constexpr (S > 1) {
     // (m, sum, acc) of every group but the head's first, then merged by it

@@ -63,6 +63,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     }
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
+      if (s0 + j >= np) break;       // (0 x infinity: weight 0 won't do)
       const float m_new = fmaxf(m, l[j]);
       const float m_use = m_new == -INFINITY ? 0.0f : m_new;
       const float keep = fast_exp2((m - m_use) * kLog2e);
