@@ -22,6 +22,10 @@ def _ptr(t):
 
 
 def _stream(dev):
+    # the current stream's handle without a Stream object around it (0.1 us
+    # against 1.9 us of a small call's host time)
+    if dev.type == "cuda" and dev.index is not None:
+        return torch._C._cuda_getCurrentRawStream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
 
 
