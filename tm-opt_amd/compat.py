@@ -154,8 +154,8 @@ def _kv_pair(k, v):
     if (not k_ok and not v_ok and k.is_cuda and kt.stride(1) == 1 and
             vt.stride(1) == 1 and kt.shape[3] == attn.HEAD_DIM and
             kt.dtype == vt.dtype == torch.bfloat16 and
-            kt.shape == vt.shape and kt.device == vt.device and 0 < kt.shape[0] <= 65535 and
-            0 < kt.shape[2] <= 32767):
+            kt.shape == vt.shape and kt.device == vt.device and
+            0 < kt.shape[0] <= 65535 and 0 < kt.shape[2] <= 32767):
         return attn._pack_rows(kt, vt)
     return (kt if k_ok else kt.contiguous(), vt if v_ok else vt.contiguous())
 

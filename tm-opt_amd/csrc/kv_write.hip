@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256) void kv_write_paged_cm_kernel(
 // writing whole 256-byte rows. LDS rows (one token) are 130 elements apart, so
 // the two-byte writes of a wave (64 tokens of one dim, 65 dwords apart) spread
 // over all banks. Two tensors of 777 tokens, 8 heads: 15.3 us for two strided
-// copies, PACKUS here.
+// copies, 4.9 us here.
 constexpr int kPackTok = 64;
 constexpr int kPackRow = 130;
 __global__ __launch_bounds__(256) void pack_rows_kernel(
@@ -314,7 +314,8 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(
 __global__ __launch_bounds__(256) void chunk_tables_kernel(
     const int64_t* __restrict__ table_dev, int64_t row_stride, int64_t rows,
     const int64_t* __restrict__ slots, int n_slots,
-    const int64_t* __restrict__ prior, int n_prior, int width, int32_t* __restrict__ table, int32_t* __restrict__ start,
+    const int64_t* __restrict__ prior, int n_prior, int width,
+    int32_t* __restrict__ table, int32_t* __restrict__ start,
     int32_t* __restrict__ cu, int total) {
   const int b = blockIdx.y;
   const int i = blockIdx.x * 256 + threadIdx.x;

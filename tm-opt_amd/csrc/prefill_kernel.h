@@ -349,22 +349,30 @@ __device__ __forceinline__ void rows_to_lds(uint32_t ob, int lane, int c,
            u32x2{pack_bf16x2(f32_to_bf16_bits(x0), f32_to_bf16_bits(x1)),
                  pack_bf16x2(f32_to_bf16_bits(x2), f32_to_bf16_bits(x3))});
 }
-// Chunk c16 of row r from there to the output (a store instruction covers 4
-// complete rows: 16 lanes x 16 bytes each).
-__device__ __forceinline__ void row_from_lds(const PrefillArgs& a, uint32_t ob,
-                                             int r, int c16, int qrow0, int len,
-                                             int t0, int head) {
-  const bool al16 = ((a.o_st | a.o_sh) & 7) == 0 && ((uintptr_t)a.out & 15) == 0;
-  const u32x4 x = __builtin_bit_cast(
-      u32x4, lds_ld128(ob + r * kRowB + 16 * (c16 ^ (r & 15))));
-  if (qrow0 + r < len) {
-    __bf16* const dst = a.out + (int64_t)(t0 + qrow0 + r) * a.o_st +
-                        (int64_t)head * a.o_sh + 8 * c16;
-    if (al16) {
-      *reinterpret_cast<u32x4*>(dst) = x;
-    } else {
-      reinterpret_cast<u32x2*>(dst)[0] = u32x2{x[0], x[1]};
-      reinterpret_cast<u32x2*>(dst)[1] = u32x2{x[2], x[3]};
+// Rows r0, r0 + STEP, ... (N of them) from there to the output, 16-byte chunk
+// c16 of each (a store instruction covers 4 complete rows: 16 lanes x 16 bytes
+// each). The loop is in here because the compiler does not take a row's
+// alignment test out of a caller's unrolled loop (8 tests per item).
+template <int N, int STEP>
+__device__ __forceinline__ void rows_from_lds(const PrefillArgs& a, uint32_t ob,
+                                              int r0, int c16, int qrow0,
+                                              int len, int t0, int head) {
+  const bool al16 = ((a.o_st | a.o_sh) & 7) == 0 &&
+                    ((uintptr_t)a.out & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int r = STEP * i + r0;
+    const u32x4 x = __builtin_bit_cast(
+        u32x4, lds_ld128(ob + r * kRowB + 16 * (c16 ^ (r & 15))));
+    if (qrow0 + r < len) {
+      __bf16* const dst = a.out + (int64_t)(t0 + qrow0 + r) * a.o_st +
+                          (int64_t)head * a.o_sh + 8 * c16;
+      if (al16) {
+        *reinterpret_cast<u32x4*>(dst) = x;
+      } else {
+        reinterpret_cast<u32x2*>(dst)[0] = u32x2{x[0], x[1]};
+        reinterpret_cast<u32x2*>(dst)[1] = u32x2{x[2], x[3]};
+      }
     }
   }
 }
@@ -1181,9 +1189,10 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
   const float l_tot = l_part + __shfl_xor(l_part, 32);
   const float inv = rejected ? __builtin_nanf("") :
                     l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  const float lse = rejected ? __builtin_nanf("") :
-                    l_tot > 0.0f ? (m_run + fast_log2(l_tot)) * kLn2
-                                 : -INFINITY;
+  auto lse = [&] {
+    return rejected ? __builtin_nanf("") :
+           l_tot > 0.0f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
+  };
   if (PART && part_slot >= 0) {
     // lane-major partial: every store writes 1 KB
     const int64_t pw = (int64_t)part_slot * 8 + w;
@@ -1195,11 +1204,11 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
         *reinterpret_cast<f32x4*>(po + (4 * db + g4) * 256) =
             f32x4{o_acc[db][4 * g4] * inv, o_acc[db][4 * g4 + 1] * inv,
                   o_acc[db][4 * g4 + 2] * inv, o_acc[db][4 * g4 + 3] * inv};
-    if (h2 == 0) a.part_lse[pw * 32 + l32] = lse;
+    if (h2 == 0) a.part_lse[pw * 32 + l32] = lse();
     return;
   }
   if (a.lse && h2 == 0 && qok)
-    a.lse[(int64_t)head * wk.total + t0 + qi] = lse;
+    a.lse[(int64_t)head * wk.total + t0 + qi] = lse();
   // O^T goes through LDS (free after the last barrier) so that the global
   // stores are whole rows.
   const uint32_t ob = lds0 + (uint32_t)w * (32 * kRowB);
@@ -1212,9 +1221,7 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
                   o_acc[db][4 * g4 + 3] * inv);
   wave_lds_sync();
   const int qrow0 = q0 + 32 * (w % QSUB);   // query of the block's row 0
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    row_from_lds(a, ob, 4 * i + (lane >> 4), lane & 15, qrow0, len, t0, head);
+  rows_from_lds<8, 4>(a, ob, lane >> 4, lane & 15, qrow0, len, t0, head);
 }
 
 template <int REP, bool REL, int SRC>

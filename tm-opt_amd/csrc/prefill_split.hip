@@ -89,10 +89,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     rows_to_lds(ob, lane, 4 * db + g4, acc[g4][0] * inv, acc[g4][1] * inv,
                 acc[g4][2] * inv, acc[g4][3] * inv);
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    row_from_lds(a, ob, 16 * i + 4 * db + (lane >> 4), lane & 15, qrow0, wk.len,
-                 wk.t0, head);
+  rows_from_lds<2, 16>(a, ob, 4 * db + (lane >> 4), lane & 15, qrow0, wk.len,
+                       wk.t0, head);
 }
 
 template <int REP, bool REL>
