@@ -337,53 +337,24 @@ __device__ __forceinline__ int cm_sig(int r) {
   return ((x & 1) << 2) | (x >> 1);
 }
 
-// A 32-row block of outputs on its way through LDS, query-major: 256-byte
-// rows, 16-byte chunks swizzled by row & 15, so neither the 8-byte writes nor
-// the 16-byte reads conflict. Chunk c (dims 8c..8c+7) of row lane & 31, half
-// lane >> 5, from four fp32 values.
-__device__ __forceinline__ void rows_to_lds(uint32_t ob, int lane, int c,
-                                            float x0, float x1, float x2,
-                                            float x3) {
-  const int r = lane & 31;
-  lds_st64(ob + r * kRowB + 16 * (c ^ (r & 15)) + 8 * (lane >> 5),
-           u32x2{pack_bf16x2(f32_to_bf16_bits(x0), f32_to_bf16_bits(x1)),
-                 pack_bf16x2(f32_to_bf16_bits(x2), f32_to_bf16_bits(x3))});
-}
-// Rows r0, r0 + STEP, ... (N of them) from there to the output, 16-byte chunk
-// c16 of each (a store instruction covers 4 complete rows: 16 lanes x 16 bytes
-// each). The loop is in here because the compiler does not take a row's
-// alignment test out of a caller's unrolled loop (8 tests per item).
-template <int N, int STEP>
-__device__ __forceinline__ void rows_from_lds(const PrefillArgs& a, uint32_t ob,
-                                              int r0, int c16, int qrow0,
-                                              int len, int t0, int head) {
-  const bool al16 = ((a.o_st | a.o_sh) & 7) == 0 &&
-                    ((uintptr_t)a.out & 15) == 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int r = STEP * i + r0;
-    const u32x4 x = __builtin_bit_cast(
-        u32x4, lds_ld128(ob + r * kRowB + 16 * (c16 ^ (r & 15))));
-    if (qrow0 + r < len) {
-      __bf16* const dst = a.out + (int64_t)(t0 + qrow0 + r) * a.o_st +
-                          (int64_t)head * a.o_sh + 8 * c16;
-      if (al16) {
-        *reinterpret_cast<u32x4*>(dst) = x;
-      } else {
-        reinterpret_cast<u32x2*>(dst)[0] = u32x2{x[0], x[1]};
-        reinterpret_cast<u32x2*>(dst)[1] = u32x2{x[2], x[3]};
-      }
-    }
-  }
-}
-
-// A work item, or (PART) a piece of it: key tiles [tile0, tile1), the result to
-// slot `part_slot` (negative: the piece is the whole item).
-template <int REP, bool REL, int SRC, bool PART>
+// One work item. Compiled twice: prefill.hip holds the kernel of whole items,
+// prefill_split.hip (TMOPT_PREFILL_PIECES) the same as a function of its split
+// kernel, over key tiles [tile0, tile1) of the item, with the result to slot
+// `part_slot` (negative: the piece is the whole item). The preprocessor keeps
+// the two apart, and not a template flag, because the pieces must not change
+// the instructions of a whole item: as one function with a flag these came
+// out in another order, and eight prompts of 512-8192 tokens (32Q/4KV) took
+// 1037 us against 1030.
+#ifdef TMOPT_PREFILL_PIECES
+template <int REP, bool REL, int SRC>
 __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
                                              const Work& wk, int item_k_lo,
                                              int tile0, int tile1,
                                              int part_slot) {
+#else
+template <int REP, bool REL, int SRC>
+__global__ __launch_bounds__(512) void prefill_kernel(PrefillArgs a) {
+#endif
   constexpr bool CM = SRC == kPackedCM;   // channel-major k / v tiles
   constexpr bool POOL = SRC == kPaged || SRC == kMixed;  // keys from pools
   constexpr bool OWN = SRC != kPaged;     // the run's keys from packed k/v
@@ -396,6 +367,10 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int h2 = lane >> 5;       // lane half
+#ifndef TMOPT_PREFILL_PIECES
+  const Work wk = schedule(a, BQ, lane, blockIdx.x);
+  if (wk.seq < 0) return;
+#endif
   const int kvh = wk.kvh;
   const int kvs = kvh / a.kv_div;   // the stored KV head its keys come from
   const int seq = wk.seq;
@@ -411,10 +386,16 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
   const int pos_hi = prior + q0 + qn - 1;     // last valid query position
   // first key any query of the block may see
   const int kwin = a.window > 0 ? max(0, pos_lo - a.window + 1) : 0;
+#ifdef TMOPT_PREFILL_PIECES
   const int k_lo = item_k_lo + tile0 * kBN;
-  const int k_hi = PART ? min(pos_hi + 1, item_k_lo + tile1 * kBN)
-                        : pos_hi + 1;         // exclusive
-  const int ntiles = PART ? tile1 - tile0 : (k_hi - k_lo + kBN - 1) / kBN;
+  const int k_hi = min(pos_hi + 1, item_k_lo + tile1 * kBN);   // exclusive
+  const int ntiles = tile1 - tile0;
+#else
+  // (tiles start at a multiple of the tile width)
+  const int k_lo = (kwin / kBN) * kBN;
+  const int k_hi = pos_hi + 1;                // exclusive
+  const int ntiles = (k_hi - k_lo + kBN - 1) / kBN;
+#endif
 
   // ---- this wave's row block: head and 32-query sub-block ----------------
   const int head = kvh * REP + w / QSUB;
@@ -1189,11 +1170,8 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
   const float l_tot = l_part + __shfl_xor(l_part, 32);
   const float inv = rejected ? __builtin_nanf("") :
                     l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  auto lse = [&] {
-    return rejected ? __builtin_nanf("") :
-           l_tot > 0.0f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
-  };
-  if (PART && part_slot >= 0) {
+#ifdef TMOPT_PREFILL_PIECES
+  if (part_slot >= 0) {
     // lane-major partial: every store writes 1 KB
     const int64_t pw = (int64_t)part_slot * 8 + w;
     float* const po = a.part_o + (pw * 16 * 64 + lane) * 4;
@@ -1204,33 +1182,57 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a,
         *reinterpret_cast<f32x4*>(po + (4 * db + g4) * 256) =
             f32x4{o_acc[db][4 * g4] * inv, o_acc[db][4 * g4 + 1] * inv,
                   o_acc[db][4 * g4 + 2] * inv, o_acc[db][4 * g4 + 3] * inv};
-    if (h2 == 0) a.part_lse[pw * 32 + l32] = lse();
+    if (h2 == 0)
+      a.part_lse[pw * 32 + l32] =
+          rejected ? __builtin_nanf("") :
+          l_tot > 0.0f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
     return;
   }
+#endif
   if (a.lse && h2 == 0 && qok)
-    a.lse[(int64_t)head * wk.total + t0 + qi] = lse();
+    a.lse[(int64_t)head * wk.total + t0 + qi] =
+        rejected ? __builtin_nanf("") :
+        l_tot > 0.0f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
   // O^T goes through LDS (free after the last barrier) so that the global
-  // stores are whole rows.
+  // stores are whole rows: the wave writes its 32 x 128 block query-major
+  // (256-byte rows, 16-byte chunks swizzled by row & 15, so neither the
+  // 8-byte writes nor the 16-byte reads conflict), then each store
+  // instruction covers 4 complete rows (16 lanes x 16 bytes per row)
+  // instead of 16 bytes of 32 rows.
   const uint32_t ob = lds0 + (uint32_t)w * (32 * kRowB);
 #pragma unroll
   for (int db = 0; db < 4; ++db)
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4)
-      rows_to_lds(ob, lane, 4 * db + g4, o_acc[db][4 * g4] * inv,
-                  o_acc[db][4 * g4 + 1] * inv, o_acc[db][4 * g4 + 2] * inv,
-                  o_acc[db][4 * g4 + 3] * inv);
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const uint32_t w0 = pack_bf16x2(f32_to_bf16_bits(o_acc[db][4 * g4] * inv),
+                                      f32_to_bf16_bits(o_acc[db][4 * g4 + 1] * inv));
+      const uint32_t w1 = pack_bf16x2(f32_to_bf16_bits(o_acc[db][4 * g4 + 2] * inv),
+                                      f32_to_bf16_bits(o_acc[db][4 * g4 + 3] * inv));
+      const int c = 4 * db + g4;    // 16-byte chunk: dims 8c .. 8c+7
+      lds_st64(ob + l32 * kRowB + 16 * (c ^ (l32 & 15)) + 8 * h2,
+               u32x2{w0, w1});
+    }
   wave_lds_sync();
   const int qrow0 = q0 + 32 * (w % QSUB);   // query of the block's row 0
-  rows_from_lds<8, 4>(a, ob, lane >> 4, lane & 15, qrow0, len, t0, head);
-}
-
-template <int REP, bool REL, int SRC>
-__global__ __launch_bounds__(512) void prefill_kernel(PrefillArgs a) {
-  constexpr int BQ = 256 / REP;
-  const Work wk = schedule(a, BQ, threadIdx.x & 63, blockIdx.x);
-  if (wk.seq < 0) return;
-  const Tiles tl = item_tiles(a, BQ, wk.prior, wk.len, wk.qb);
-  prefill_item<REP, REL, SRC, false>(a, wk, tl.k_lo, 0, tl.n, 0);
+  const int c16 = lane & 15;
+  const bool al16 = ((a.o_st | a.o_sh) & 7) == 0 &&
+                    ((uintptr_t)a.out & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 4 * i + (lane >> 4);
+    const u32x4 x = __builtin_bit_cast(
+        u32x4, lds_ld128(ob + r * kRowB + 16 * (c16 ^ (r & 15))));
+    if (qrow0 + r < len) {
+      __bf16* const dst = a.out + (int64_t)(t0 + qrow0 + r) * a.o_st +
+                          (int64_t)head * a.o_sh + 8 * c16;
+      if (al16) {
+        *reinterpret_cast<u32x4*>(dst) = x;
+      } else {
+        reinterpret_cast<u32x2*>(dst)[0] = u32x2{x[0], x[1]};
+        reinterpret_cast<u32x2*>(dst)[1] = u32x2{x[2], x[3]};
+      }
+    }
+  }
 }
 
 }  // namespace

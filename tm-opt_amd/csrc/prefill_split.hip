@@ -1,5 +1,6 @@
 // Prefill launches whose keys are split over work-groups (see key_pieces in
 // prefill_kernel.h): the split kernel and the merge of its pieces.
+#define TMOPT_PREFILL_PIECES
 #include "prefill_kernel.h"
 
 namespace tmopt {
@@ -20,11 +21,50 @@ __global__ __launch_bounds__(512) void prefill_split_kernel(PrefillArgs a) {
   const int slot = pc.nall > 1 ? (int)blockIdx.x : -1;
   if constexpr (REL) {
     if (level < pc.np && pc.nall > 1) {
-      prefill_item<REP, false, SRC, true>(a, wk, tl.k_lo, t0, t1, slot);
+      prefill_item<REP, false, SRC>(a, wk, tl.k_lo, t0, t1, slot);
       return;
     }
   }
-  prefill_item<REP, REL, SRC, true>(a, wk, tl.k_lo, t0, t1, slot);
+  prefill_item<REP, REL, SRC>(a, wk, tl.k_lo, t0, t1, slot);
+}
+
+// A 32-row block of outputs on its way through LDS, query-major: 256-byte
+// rows, 16-byte chunks swizzled by row & 15, so neither the 8-byte writes nor
+// the 16-byte reads conflict. Chunk c (dims 8c..8c+7) of row lane & 31, half
+// lane >> 5, from four fp32 values.
+__device__ __forceinline__ void rows_to_lds(uint32_t ob, int lane, int c,
+                                            float x0, float x1, float x2,
+                                            float x3) {
+  const int r = lane & 31;
+  lds_st64(ob + r * kRowB + 16 * (c ^ (r & 15)) + 8 * (lane >> 5),
+           u32x2{pack_bf16x2(f32_to_bf16_bits(x0), f32_to_bf16_bits(x1)),
+                 pack_bf16x2(f32_to_bf16_bits(x2), f32_to_bf16_bits(x3))});
+}
+// Rows r0, r0 + STEP, ... (N of them) from there to the output, 16-byte chunk
+// c16 of each (a store instruction covers 4 complete rows: 16 lanes x 16 bytes
+// each).
+template <int N, int STEP>
+__device__ __forceinline__ void rows_from_lds(const PrefillArgs& a, uint32_t ob,
+                                              int r0, int c16, int qrow0,
+                                              int len, int t0, int head) {
+  const bool al16 = ((a.o_st | a.o_sh) & 7) == 0 &&
+                    ((uintptr_t)a.out & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int r = STEP * i + r0;
+    const u32x4 x = __builtin_bit_cast(
+        u32x4, lds_ld128(ob + r * kRowB + 16 * (c16 ^ (r & 15))));
+    if (qrow0 + r < len) {
+      __bf16* const dst = a.out + (int64_t)(t0 + qrow0 + r) * a.o_st +
+                          (int64_t)head * a.o_sh + 8 * c16;
+      if (al16) {
+        *reinterpret_cast<u32x4*>(dst) = x;
+      } else {
+        reinterpret_cast<u32x2*>(dst)[0] = u32x2{x[0], x[1]};
+        reinterpret_cast<u32x2*>(dst)[1] = u32x2{x[2], x[3]};
+      }
+    }
+  }
 }
 
 // Combine the pieces of the items that were split: grid (n_base, 8), one
