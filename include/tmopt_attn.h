@@ -454,7 +454,7 @@ int tmopt_attn_prefill_varlen_split(
  * Bytes of workspace tmopt_attn_prefill_varlen_split needs for a launch shape
  * on the current device; 0 where it does not split (bt_stride 0 without a
  * block table). It does not depend on the lengths, which only the device
- * knows: at most 2 x 129 KB per compute unit plus one round of query blocks.
+ * knows: at most 2 x 129 KB per compute unit and a count per query block.
  */
 size_t tmopt_attn_prefill_workspace_size(int num_seqs, int max_seqlen_q,
                                          int HQ, int HKV, int64_t bt_stride,

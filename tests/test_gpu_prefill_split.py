@@ -138,6 +138,33 @@ def test_split_repeats_bitwise_and_matches_one_launch(tm, dev):
     assert e.value.status == tm._lib.TMOPT_EWORKSPACE
 
 
+@pytest.mark.parametrize("lens,prior", [
+    ([64, 256], [7936, 7680]), ([96, 256], [7808, 6720]), ([7], [40])])
+def test_merge_reads_what_was_written(tm, dev, lens, prior):
+    """Lengths at which the fp32 rule for the number of pieces sits on a
+    rounding edge (12 or 13 of them with and without an fma; found with both
+    forms on the CPU), and a launch whose items all stay whole, over a scratch
+    full of NaN: the merge takes exactly the pieces that were left for it."""
+    wl = import_module("tm-opt_amd.workloads")
+    a = _runs(lens, prior, 16, 2, 64, "paged", wl)
+    if lens == [7]:
+        a["block_table"] = torch.nn.functional.pad(a["block_table"], (0, 100))
+    real, held = tm._lib.call, []
+
+    def call(name, *x):
+        if name.endswith("_split"):
+            held.append(torch.full((x[-2] // 4 + 4,), float("nan"),
+                                   device=dev))
+            x = x[:-3] + (held[0].data_ptr(),) + x[-2:]
+        return real(name, *x)
+    tm._lib.call = call
+    try:
+        _check(tm, dev, a, f"{lens} after {prior}")
+    finally:
+        tm._lib.call = real
+    assert held
+
+
 @pytest.mark.parametrize("prior", [1500, 4000])
 def test_infinite_values(tm, dev, prior):
     """An infinity in V that every query sees, in the last piece, is one in

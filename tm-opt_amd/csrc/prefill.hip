@@ -66,6 +66,9 @@ int split_levels(int64_t n_base, int BQ, int max_seqlen, int64_t bt_stride,
 }
 
 constexpr int64_t kSlotBytes = (256 * kD + 256) * sizeof(float);
+int64_t workspace_bytes_of(int levels, int64_t n_base) {
+  return levels * n_base * kSlotBytes + ((n_base * 4 + 15) & ~(int64_t)15);
+}
 
 template <int REP>
 void launch(const PrefillArgs& a, int src, size_t lds, hipStream_t st) {
@@ -133,7 +136,7 @@ extern "C" size_t tmopt_attn_prefill_workspace_size(int num_seqs,
   const int64_t n = level_wgs((int)hkv, bq, num_seqs, max_seqlen_q);
   const int levels =
       split_levels(n, bq, max_seqlen_q, bt_stride, table_wrap, window);
-  return levels > 1 ? (size_t)(levels * n * kSlotBytes) : 0;
+  return levels > 1 ? (size_t)workspace_bytes_of(levels, n) : 0;
 }
 
 static int prefill_impl(
@@ -320,14 +323,15 @@ static int prefill_impl(
                  : split_levels(a.n_base, 256 / rep, max_seqlen_q,
                                 pooled ? bt_stride : 0, table_wrap, window);
   const int64_t slots = (int64_t)a.nsplit * a.n_base;
-  TMOPT_REQUIRE(a.nsplit <= 1 ||
-                    ((int64_t)workspace_bytes >= slots * kSlotBytes &&
-                     (uintptr_t)workspace % 16 == 0),
+  const int64_t need = workspace_bytes_of(a.nsplit, a.n_base);
+  TMOPT_REQUIRE(a.nsplit <= 1 || ((int64_t)workspace_bytes >= need &&
+                                  (uintptr_t)workspace % 16 == 0),
                 TMOPT_EWORKSPACE,
                 "prefill: workspace %zu bytes < %lld needed (or unaligned)",
-                workspace_bytes, (long long)(slots * kSlotBytes));
+                workspace_bytes, (long long)need);
   a.part_o = (float*)workspace;
   a.part_lse = a.part_o + slots * 256 * kD;
+  a.part_n = (int*)(a.part_lse + slots * 256);
   a.nqb_max = (max_seqlen_q + 256 / rep - 1) / (256 / rep);
   hipStream_t st = (hipStream_t)stream;
   const size_t lds = kNStage * kStage + (a.rel ? 8 * kBiasB : 0);

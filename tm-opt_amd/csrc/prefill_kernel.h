@@ -94,6 +94,7 @@ struct PrefillArgs {
   int split_wgs;     // work-groups to aim at: the compute units
   float* part_o;     // [nsplit * n_base][8 waves][16][64 lanes][4] fp32
   float* part_lse;   // [nsplit * n_base][256 rows]
+  int* part_n;       // [n_base] pieces of each item (0: no such item)
 };
 
 // prefill_split.hip: the split kernel and the merge, for `rep` query heads per
@@ -244,8 +245,7 @@ __device__ __forceinline__ Tiles item_tiles(const PrefillArgs& a, int BQ,
 // in piece order. An item gets as many pieces as compute units by its share of
 // the launch's tiles (rounded down, so that the pieces run in one wave; a
 // share a little short of a whole one counts as one: the tiles of the launch
-// are an estimate from the first and last block of each run, the same in both
-// kernels), each of kMinPiece tiles at least, and stays whole where the pieces'
+// are an estimate from the first and last block of each run), each of kMinPiece tiles at least, and stays whole where the pieces'
 // cost (~6 us for their start and the merge, 0.065 us for the 129 KB that each
 // piece of the launch writes and reads back) is above the tiles saved, 1.7 us
 // each.

@@ -6,17 +6,27 @@
 namespace tmopt {
 namespace {
 
-// prefill_kernel with split keys (items that stay whole included).
+// prefill_kernel with split keys (items that stay whole included). The number
+// of pieces goes to the merge through memory: it comes of fp32 arithmetic next
+// to rounding edges, which another kernel need not contract the same way (fma
+// or not, 64 + 256 queries after 7,936 and 7,680 keys give 12 or 13 pieces),
+// and the merge must read exactly the slots that were written. Every work-group
+// of this kernel runs the same instructions on the same lengths.
 template <int REP, bool REL, int SRC>
 __global__ __launch_bounds__(512) void prefill_split_kernel(PrefillArgs a) {
   constexpr int BQ = 256 / REP;
   const int lane = threadIdx.x & 63;
   const int level = (int)blockIdx.x / a.n_base;
-  const Work wk = schedule(a, BQ, lane, (int)blockIdx.x - level * a.n_base);
-  if (wk.seq < 0) return;
+  const int item = (int)blockIdx.x - level * a.n_base;
+  const Work wk = schedule(a, BQ, lane, item);
+  if (wk.seq < 0) {
+    if (level == 0 && threadIdx.x == 0) a.part_n[item] = 0;
+    return;
+  }
   const Tiles tl = item_tiles(a, BQ, wk.prior, wk.len, wk.qb);
   const Pieces pc = key_pieces(a, BQ, lane, wk, tl);
   if (level >= pc.nall) return;
+  if (level == 0 && threadIdx.x == 0) a.part_n[item] = pc.nall;
   const int t0 = pc.begin(level, tl.n), t1 = pc.begin(level + 1, tl.n);
   const int slot = pc.nall > 1 ? (int)blockIdx.x : -1;
   if constexpr (REL) {
@@ -77,11 +87,9 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const int lane = threadIdx.x & 63;
   const int db = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l32 = lane & 31;
+  const int np = min(as_const(a.part_n)[blockIdx.x], a.nsplit);
+  if (np <= 1) return;                        // no item, or written in place
   const Work wk = schedule(a, BQ, lane, blockIdx.x);
-  if (wk.seq < 0) return;
-  const Tiles tl = item_tiles(a, BQ, wk.prior, wk.len, wk.qb);
-  const int np = key_pieces(a, BQ, lane, wk, tl).nall;
-  if (np <= 1) return;                        // written in place
   const int w = blockIdx.y;                   // row block = wave of the item
   const int qrow0 = wk.qb * BQ + 32 * (w % QSUB);
   const int head = wk.kvh * REP + w / QSUB;
