@@ -154,3 +154,57 @@ def test_bench_fails_loudly_without_a_gpu():
     assert r.returncode == 1
     assert "no GPU" in r.stderr
     assert r.stdout.strip() == ""
+
+
+@pytest.mark.parametrize("n,T,split", [(0, 64, False), (300, 64, False),
+                                       (896, 64, False), (897, 64, True),
+                                       (2000, 16, True)])
+def test_split_follows_the_context_and_not_the_table(tm, monkeypatch, n, T,
+                                                     split):
+    """A short chunk under a page table as wide as the pool is one launch
+    where the host knows its context (960 keys, 15 tiles, are not split, 961
+    are): through prefill_chunk_state, which knows it, and the calls that can
+    be told. Without the bound the table's width decides."""
+    attn = import_module("tm-opt_amd.attn")
+    compat = import_module("tm-opt_amd.compat")
+    scratch = []
+
+    def call(name, *args):
+        if name.endswith("_split"):
+            scratch.append(args[-2])
+    monkeypatch.setattr(tm._lib, "call", call)
+    monkeypatch.setattr(attn, "_stream", lambda dev: None)
+    bf = torch.bfloat16
+    hq, hkv, pages = 16, 2, 500
+    q, k = torch.zeros((T, hq, 128), dtype=bf), torch.zeros((T, hkv, 128),
+                                                            dtype=bf)
+    pool = torch.zeros((8, 16, hkv, 128), dtype=bf)
+
+    class Paged:
+        kp = vp = pool
+        page_size = 16
+        table_dev_row = torch.zeros(pages, dtype=torch.int64)
+
+        def ensure_pages(self, last):
+            pass
+    c = Paged()
+    c.n = n
+    compat.prefill_chunk_state(q, k, k, None, c)
+    assert c.n == n + T
+    i64 = lambda x: torch.tensor([x])           # noqa: E731
+    table = torch.zeros((1, pages), dtype=torch.int64)
+    for bound in (n + T, None):
+        compat.attn_prefill_chunk_global(q, k, k, None, pool, pool, table,
+                                         i64(0), i64(n), max_context=bound)
+        tm.prefill_varlen(q, None, None,
+                          torch.tensor([0, T], dtype=torch.int32), 0.1,
+                          max_seqlen=T, k_pool=pool, v_pool=pool,
+                          prior_lens=torch.tensor([n], dtype=torch.int32),
+                          block_table=table.int(), max_context=bound)
+    assert [s > 0 for s in scratch] == [split] * 3 + [True] * 2
+    ring = torch.zeros((2, 1280, hkv, 128), dtype=bf)
+    del scratch[:]
+    for bound in (n + T, None):
+        compat.attn_prefill_chunk_swa(q, k, k, None, ring, ring, i64(0),
+                                      i64(n), max_context=bound)
+    assert [s > 0 for s in scratch] == [split, True]

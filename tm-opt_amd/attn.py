@@ -428,7 +428,7 @@ def _prefill_workspace_size(device, *shape):
 def prefill_varlen(q, k, v, cu_seqlens, scale, window=0, max_seqlen=None,
                    prior_lens=None, k_pool=None, v_pool=None,
                    block_table=None, table_wrap=0, rel=None, out=None,
-                   lse=None, return_lse=True, reject=None):
+                   lse=None, return_lse=True, reject=None, max_context=None):
     """Varlen causal (optionally windowed) prefill attention on bf16 MFMA.
 
     q [total, HQ, D] bf16 (D contiguous, any token / head strides);
@@ -453,16 +453,28 @@ def prefill_varlen(q, k, v, cu_seqlens, scale, window=0, max_seqlen=None,
     pos_q - pos_k] inside 0 <= dist < E (attn_prefill.py:115-120).
     reject: optional int32 device scalar; nonzero -> NaN outputs (device-side
     input rejection without a host sync).
+    A launch of few query blocks that may see many keys splits these over
+    work-groups and merges the pieces: a second launch, up to 2 x 129 KB of
+    scratch per compute unit (66 MB), and last bits of the results that depend
+    on the launch's other runs and the table's width (a run's pieces are its
+    share of the launch). max_context: an upper bound of prior + run length
+    over the runs, where the host has one; without it the row width of the
+    block table bounds the keys, and short contexts under a wide table pay for
+    the launch that merges nothing (graph replays, 64Q/8KV, 4,096 pages: 64
+    tokens without context 10.0 us against 7.5, 500 23.4 against 20.8). It
+    decides about the split alone.
     Returns (out [total, HQ, D] bf16, lse [HQ, total] fp32 or None).
     Reference: engine/pyengine/kernels/attn_prefill.py:71-194."""
     return _prefill_varlen(q, k, v, cu_seqlens, scale, window, max_seqlen,
                            prior_lens, k_pool, v_pool, block_table,
-                           table_wrap, rel, out, lse, return_lse, reject)
+                           table_wrap, rel, out, lse, return_lse, reject,
+                           max_context)
 
 
 def _prefill_varlen(q, k, v, cu_seqlens, scale, window, max_seqlen,
                     prior_lens, k_pool, v_pool, block_table, table_wrap, rel,
-                    out, lse, return_lse, reject, split=True):
+                    out, lse, return_lse, reject, max_context=None,
+                    split=True):
     """prefill_varlen; split False: one launch, for a caller that fills the
     rest of the device with other work."""
     total, HQ, D = q.shape
@@ -533,8 +545,13 @@ def _prefill_varlen(q, k, v, cu_seqlens, scale, window, max_seqlen,
     # scratch for the pieces of a launch too small for the device (0 bytes
     # for any other): the kernel splits its keys
     bts = block_table.stride(0) if pooled else 0
-    n = _prefill_workspace_size(dev.index, S, int(max_seqlen), HQ, HKV, bts,
-                                int(table_wrap), int(window)) if split else 0
+    n = 0
+    if split and (max_context is None or not pooled or _prefill_workspace_size(
+            dev.index, S, int(max_seqlen), HQ, HKV,
+            max(1, -(-(int(max_context) - int(max_seqlen)) // page_size)), 0,
+            int(window))):
+        n = _prefill_workspace_size(dev.index, S, int(max_seqlen), HQ, HKV,
+                                    bts, int(table_wrap), int(window))
     ws = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
     _lib.call("tmopt_attn_prefill_varlen_split", _ptr(q), q.stride(0),
               q.stride(1),

@@ -393,7 +393,8 @@ def _chunk_max(q, cu_seqlens, max_seqlen):
 
 
 def attn_prefill_chunk_swa(q, k, v, rel, pool_k, pool_v, slots, prior,
-                           cu_seqlens=None, max_seqlen=None):
+                           cu_seqlens=None, max_seqlen=None,
+                           max_context=None):
     """Chunked prefill of a sliding-window layer over SwaPool ring rows.
 
     q [total, H, D], k/v [total, HK, D] bf16: the chunks of B sequences
@@ -403,7 +404,8 @@ def attn_prefill_chunk_swa(q, k, v, rel, pool_k, pool_v, slots, prior,
     i64 tokens each ring has seen (RingKV.n). Scale 1/D. Attends, then
     appends the chunks to the rings (only the last W positions survive).
     max_seqlen: the longest chunk; with several sequences pass it to keep
-    the call free of host synchronisation (graph capture).
+    the call free of host synchronisation (graph capture). max_context: the
+    longest prior + chunk, where the host knows it (prefill_varlen's).
     Returns out [total, H, D] bf16."""
     total, H, D = q.shape
     S1, W, HK, _ = pool_k.shape
@@ -423,7 +425,8 @@ def attn_prefill_chunk_swa(q, k, v, rel, pool_k, pool_v, slots, prior,
     out, _ = attn.prefill_varlen(q, k, v, cu, 1.0 / D, window=W,
                                  max_seqlen=max_seqlen, prior_lens=start,
                                  k_pool=kp, v_pool=vp, block_table=table,
-                                 table_wrap=per, rel=rel, return_lse=False)
+                                 table_wrap=per, rel=rel, return_lse=False,
+                                 max_context=max_context)
     attn.kv_write_paged(k, v, table, start, kp, vp, cu_seqlens=cu,
                         max_seqlen=max_seqlen, table_wrap=per)
     return out
@@ -431,7 +434,7 @@ def attn_prefill_chunk_swa(q, k, v, rel, pool_k, pool_v, slots, prior,
 
 def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
                               slots, prior, cu_seqlens=None,
-                              max_seqlen=None):
+                              max_seqlen=None, max_context=None):
     """Chunked prefill of a global layer over GlobalPool pages.
 
     q [total, H, D], k/v [total, HK, D] bf16 packed by cu_seqlens [B+1]
@@ -442,7 +445,9 @@ def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
     [B] i64; prior [B] i64 (PagedKV.n). Scale 1/D, causal. Attends, then
     appends the chunks through the page table. max_seqlen: the longest
     chunk; with several sequences pass it to keep the call free of host
-    synchronisation (graph capture). Returns out [total, H, D]."""
+    synchronisation (graph capture). max_context: the longest prior + chunk,
+    where the host knows it (prefill_varlen's: the page table's width says
+    nothing about it). Returns out [total, H, D]."""
     total, H, D = q.shape
     assert pool_kp.is_contiguous() and pool_vp.is_contiguous()
     assert pool_kp.shape[1] == PAGE
@@ -462,7 +467,7 @@ def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
                                  max_seqlen=max_seqlen, prior_lens=start,
                                  k_pool=pool_kp, v_pool=pool_vp,
                                  block_table=table, rel=rel,
-                                 return_lse=False)
+                                 return_lse=False, max_context=max_context)
     attn.kv_write_paged(k, v, table, start, pool_kp, pool_vp, cu_seqlens=cu,
                         max_seqlen=max_seqlen)
     return out
@@ -503,7 +508,8 @@ def prefill_chunk_state(q, k, v, rel, cache):
     out, _ = attn.prefill_varlen(q, k, v, cu, 1.0 / D, window=window,
                                  max_seqlen=T, prior_lens=prior, k_pool=kp,
                                  v_pool=vp, block_table=table,
-                                 table_wrap=wrap, rel=rel, return_lse=False)
+                                 table_wrap=wrap, rel=rel, return_lse=False,
+                                 max_context=n + T)
     attn.kv_write_paged(k, v, table, prior, kp, vp, cu_seqlens=cu,
                         max_seqlen=T, table_wrap=wrap)
     cache.n = n + T
