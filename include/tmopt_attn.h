@@ -166,13 +166,16 @@ int tmopt_pack_rows(const void* k, int64_t k_stride_row, int64_t k_stride_head,
  * int64 at stride table_stride; NULL: slots[b] * width + i, a SwaPool ring of
  * width pages), start_pos[b] = prior[b] for the n_prior runs and, if cu_seqlens is not NULL,
  * cu_seqlens = {0, total}. A negative slot counts from the last row, as
- * torch's indexing does; a slot outside the table names no page (-1).
+ * torch's indexing does; a slot outside the table names no page (-1). reject
+ * (may be NULL) takes 1 if there is such a slot, else 0, for the prefill's
+ * argument of that name.
  */
 int tmopt_chunk_tables(const int64_t* table_dev, int64_t table_stride,
                        int64_t table_rows, const int64_t* slots,
                        int n_slots, const int64_t* prior, int n_prior,
                        int width, int32_t* block_table, int32_t* start_pos,
-                       int32_t* cu_seqlens, int total, tmopt_stream_t stream);
+                       int32_t* cu_seqlens, int total, int32_t* reject,
+                       tmopt_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Paged decode attention (split-KV + LSE combine)                          */

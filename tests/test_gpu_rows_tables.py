@@ -80,6 +80,37 @@ def test_chunk_tables_are_the_index_expressions(tm, dev, B, S, width):
     assert (table == -1).all()
 
 
+@pytest.mark.parametrize("bad", [3, -4, 1 << 40])
+@pytest.mark.parametrize("prior", [20, 1500])
+def test_slot_outside_the_table_is_rejected(tm, dev, bad, prior):
+    """A slot that names no row of the page table (torch's indexing refuses
+    it) makes the whole call NaN, in one launch and with split keys, and
+    appends nothing for it; slots that count from the end are accepted."""
+    rows, width, T = 3, 100, 8
+    g = torch.Generator().manual_seed(9)
+    r = lambda *s: torch.randn(s, generator=g).bfloat16().to(dev)  # noqa: E731
+    q, k, v = r(2 * T, 16, 128), r(2 * T, 2, 128), r(2 * T, 2, 128)
+    kp, vp = r(rows * width, 16, 2, 128), r(rows * width, 16, 2, 128)
+    td = torch.randperm(rows * width, generator=g).view(rows, width).to(dev)
+    cu = torch.tensor([0, T, 2 * T], dtype=torch.int32, device=dev)
+    pr = torch.tensor([prior, prior], device=dev)
+    for slots in ([bad, 1], [1, bad], [-rows, rows - 1]):
+        k0, v0 = kp.clone(), vp.clone()
+        out = tm.attn_prefill_chunk_global(
+            q, k, v, None, k0, v0, td, torch.tensor(slots, device=dev), pr,
+            cu_seqlens=cu, max_seqlen=T)
+        torch.cuda.synchronize()
+        if bad not in slots:
+            assert not out.isnan().any()
+            continue
+        assert out.isnan().all()
+        pages = td[1, prior // 16:(prior + T - 1) // 16 + 1]
+        same = torch.ones(rows * width, dtype=torch.bool)
+        same[pages.cpu()] = False
+        assert torch.equal(k0.cpu()[same], kp.cpu()[same])
+        assert torch.equal(v0.cpu()[same], vp.cpu()[same])
+
+
 @pytest.mark.parametrize("B,HQ,HK,W", [(1, 64, 16, 512), (38, 64, 16, 128),
                                        (39, 64, 16, 128), (73, 32, 4, 64)])
 def test_ring_grid_line(tm, dev, B, HQ, HK, W):

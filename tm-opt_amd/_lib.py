@@ -58,7 +58,7 @@ SIGNATURES = {
         _c_i32, _c_i32, _c_i32, _c_i32, _c_ptr, _c_ptr, _c_ptr]),
     "tmopt_chunk_tables": (_c_i32, [
         _c_ptr, _c_i64, _c_i64, _c_ptr, _c_i32, _c_ptr, _c_i32, _c_i32,
-        _c_ptr, _c_ptr, _c_ptr, _c_i32, _c_ptr]),
+        _c_ptr, _c_ptr, _c_ptr, _c_i32, _c_ptr, _c_ptr]),
     "tmopt_attn_decode_default_workgroups": (_c_i32, [_c_i32]),
     "tmopt_attn_decode_workspace_size": (_c_size, [
         _c_i32, _c_i32, _c_i32, _c_i32, _c_i32]),

@@ -157,26 +157,29 @@ def _pack_rows(k, v):
     return ko, vo
 
 
-def _chunk_tables(slots, prior, width, table_dev=None, total=None):
+def _chunk_tables(slots, prior, width, table_dev=None, total=None,
+                  reject=False):
     """A chunk batch's block table [slots, width], start positions (prior)
     and (with total) run bounds [2], all int32, in one launch
     (tmopt_chunk_tables): rows `slots` of table_dev, or the rings `slots` of
-    width pages."""
+    width pages. reject: a fourth tensor, int32 [1], 1 if a slot names no row
+    of table_dev, for prefill_varlen's argument."""
     assert slots.dim() == 1 and prior.dim() == 1
     assert slots.device == prior.device
     assert table_dev is None or table_dev.device == slots.device
     slots, prior = slots.contiguous(), prior.contiguous()
     B, S = slots.shape[0], prior.shape[0]
-    n = B * width
-    buf = torch.empty(n + S + 2, dtype=torch.int32, device=slots.device)
-    table, start, cu = buf[:n].view(B, width), buf[n:n + S], buf[n + S:]
+    buf = torch.empty(B * width + S + 3, dtype=torch.int32,
+                      device=slots.device)
+    table, start, cu, flag = buf.split_with_sizes([B * width, S, 2, 1])
+    table = table.view(B, width)
     _lib.call("tmopt_chunk_tables", _ptr(table_dev),
               0 if table_dev is None else table_dev.stride(0),
               0 if table_dev is None else table_dev.shape[0], _ptr(slots), B,
               _ptr(prior), S, width, _ptr(table), _ptr(start),
               None if total is None else _ptr(cu), total or 0,
-              _stream(slots.device))
-    return table, start, cu
+              _ptr(flag) if reject else None, _stream(slots.device))
+    return (table, start, cu, flag) if reject else (table, start, cu)
 
 
 # --------------------------------------------------------------------------

@@ -447,7 +447,9 @@ def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
     chunk; with several sequences pass it to keep the call free of host
     synchronisation (graph capture). max_context: the longest prior + chunk,
     where the host knows it (prefill_varlen's: the page table's width says
-    nothing about it). Returns out [total, H, D]."""
+    nothing about it). A slot outside table_dev rejects the call on the
+    device, without a host synchronisation: out is NaN, and nothing of that
+    sequence is appended. Returns out [total, H, D]."""
     total, H, D = q.shape
     assert pool_kp.is_contiguous() and pool_vp.is_contiguous()
     assert pool_kp.shape[1] == PAGE
@@ -458,16 +460,17 @@ def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
     max_seqlen = _chunk_max(q, cu_seqlens, max_seqlen)
     if table_dev.stride(1) != 1 or table_dev.stride(0) < table_dev.shape[1]:
         table_dev = table_dev.contiguous()
-    table, start, cu = attn._chunk_tables(
+    table, start, cu, reject = attn._chunk_tables(
         slots.to(table_dev.device), prior, table_dev.shape[1], table_dev,
-        total if cu_seqlens is None else None)
+        total if cu_seqlens is None else None, reject=True)
     if cu_seqlens is not None:
         cu = cu_seqlens
     out, _ = attn.prefill_varlen(q, k, v, cu, 1.0 / D, window=0,
                                  max_seqlen=max_seqlen, prior_lens=start,
                                  k_pool=pool_kp, v_pool=pool_vp,
                                  block_table=table, rel=rel,
-                                 return_lse=False, max_context=max_context)
+                                 return_lse=False, reject=reject,
+                                 max_context=max_context)
     attn.kv_write_paged(k, v, table, start, pool_kp, pool_vp, cu_seqlens=cu,
                         max_seqlen=max_seqlen)
     return out

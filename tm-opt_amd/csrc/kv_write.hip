@@ -310,15 +310,23 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(
 // table, rows x width int64), or slots[b] * ring_pages + i without one (a ring
 // of ring_pages = width pages); start[b] = prior[b]; with `cu`, one run of
 // `total` rows. A slot counts from the end if negative, as torch's indexing
-// does; the entries of one outside the table are -1 (no page).
+// does; the entries of one outside the table are -1 (no page), and `reject`
+// then holds 1 (else 0): the first work-group looks at all of them.
 __global__ __launch_bounds__(256) void chunk_tables_kernel(
     const int64_t* __restrict__ table_dev, int64_t row_stride, int64_t rows,
     const int64_t* __restrict__ slots, int n_slots,
     const int64_t* __restrict__ prior, int n_prior, int width,
     int32_t* __restrict__ table, int32_t* __restrict__ start,
-    int32_t* __restrict__ cu, int total) {
+    int32_t* __restrict__ cu, int total, int32_t* __restrict__ reject) {
   const int b = blockIdx.y;
   const int i = blockIdx.x * 256 + threadIdx.x;
+  if (reject != nullptr && blockIdx.x == 0 && b == 0) {
+    int bad = 0;
+    for (int j = threadIdx.x; table_dev != nullptr && j < n_slots; j += 256)
+      bad |= slots[j] < -rows || slots[j] >= rows;
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0) reject[0] = bad ? 1 : 0;
+  }
   if (b < n_slots && i < width) {
     int64_t s = slots[b];
     int32_t page;
@@ -568,7 +576,8 @@ extern "C" int tmopt_chunk_tables(const int64_t* table_dev,
                                   const int64_t* prior, int n_prior,
                                   int width, int32_t* block_table,
                                   int32_t* start_pos, int32_t* cu_seqlens,
-                                  int total, tmopt_stream_t stream) {
+                                  int total, int32_t* reject,
+                                  tmopt_stream_t stream) {
   clear_error();
   if (n_slots == 0 && n_prior == 0) return TMOPT_OK;
   TMOPT_REQUIRE(n_slots >= 0 && n_slots <= 65535 && n_prior >= 0 &&
@@ -586,6 +595,7 @@ extern "C" int tmopt_chunk_tables(const int64_t* table_dev,
                           (unsigned)(n_slots > n_prior ? n_slots : n_prior)),
                      dim3(256), 0, (hipStream_t)stream, table_dev,
                      table_stride, table_rows, slots, n_slots, prior, n_prior,
-                     width, block_table, start_pos, cu_seqlens, total);
+                     width, block_table, start_pos, cu_seqlens, total,
+                     reject);
   return check_launch("chunk_tables");
 }
