@@ -111,6 +111,31 @@ def test_slot_outside_the_table_is_rejected(tm, dev, bad, prior):
         assert torch.equal(v0.cpu()[same], vp.cpu()[same])
 
 
+@pytest.mark.parametrize("slots", [0, 2])
+def test_batch_of_no_chunks(tm, dev, slots):
+    """No run (cu_seqlens of one entry), with slots or without: an empty
+    output and untouched pools, as before the index tensors were one
+    launch."""
+    bf = torch.bfloat16
+    q = torch.zeros((0, 16, 128), dtype=bf, device=dev)
+    k = torch.zeros((0, 2, 128), dtype=bf, device=dev)
+    kp, vp = (torch.ones((8, 16, 2, 128), dtype=bf, device=dev)
+              for _ in range(2))
+    none = torch.zeros(0, dtype=torch.int64, device=dev)
+    sl = torch.arange(slots, device=dev)
+    kw = dict(cu_seqlens=torch.zeros(1, dtype=torch.int32, device=dev),
+              max_seqlen=0)
+    out = tm.attn_prefill_chunk_global(
+        q, k, k, None, kp, vp, torch.zeros((2, 4), dtype=torch.int64,
+                                           device=dev), sl, none, **kw)
+    assert out.shape == q.shape
+    ring = torch.ones((3, 32, 2, 128), dtype=bf, device=dev)
+    out = tm.attn_prefill_chunk_swa(q, k, k, None, ring, ring, sl, none, **kw)
+    torch.cuda.synchronize()
+    assert out.shape == q.shape
+    assert (kp == 1).all() and (vp == 1).all() and (ring == 1).all()
+
+
 @pytest.mark.parametrize("B,HQ,HK,W", [(1, 64, 16, 512), (38, 64, 16, 128),
                                        (39, 64, 16, 128), (73, 32, 4, 64)])
 def test_ring_grid_line(tm, dev, B, HQ, HK, W):

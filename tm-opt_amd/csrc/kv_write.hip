@@ -584,8 +584,9 @@ extern "C" int tmopt_chunk_tables(const int64_t* table_dev,
                     n_prior <= 65535 && width > 0,
                 TMOPT_EINVAL, "chunk_tables: slots=%d prior=%d width=%d",
                 n_slots, n_prior, width);
-  TMOPT_REQUIRE(slots && prior && block_table && start_pos, TMOPT_EINVAL,
-                "chunk_tables: null pointer");
+  TMOPT_REQUIRE((n_slots == 0 || (slots && block_table)) &&
+                    (n_prior == 0 || (prior && start_pos)),
+                TMOPT_EINVAL, "chunk_tables: null pointer");
   TMOPT_REQUIRE(table_dev == nullptr ||
                     (table_rows > 0 && table_stride >= width),
                 TMOPT_EINVAL, "chunk_tables: rows=%lld stride=%lld width=%d",
