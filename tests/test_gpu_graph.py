@@ -121,3 +121,31 @@ def test_prefill_fused_first_call_in_capture(tm, dev):
         torch.cuda.synchronize()
         del noise
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("overlap", [False, True])
+def test_mixed_step_allocates_nothing(tm, dev, overlap):
+    """A mixed step whose prefill splits its keys (two 40-token chunks after
+    2,000) runs without an allocation, the scratch of the pieces included;
+    the graph's replays equal the eager step bitwise."""
+    wl = import_module("tm-opt_amd.workloads")
+    graph = import_module("tm-opt_amd.graph")
+    step = wl.config5(dev, n_layers=4, window=1500, n_decode=5, chunk=40,
+                      prior=2000, n_chunks=2, lo=100, hi=3000)
+    m = graph.MixedStepGraph(step, overlap=overlap)
+    assert (m.ws_p.numel() > 0) != overlap
+    m.run_eager()
+    torch.cuda.synchronize()
+    stat = "allocation.all.allocated"
+    n = torch.cuda.memory_stats()[stat]
+    m.run_eager()
+    assert torch.cuda.memory_stats()[stat] == n
+    torch.cuda.synchronize()
+    want = [x.clone() for x in (m.out_p, m.out_d, m.lse_d)]
+    m.capture()
+    for _ in range(3):
+        m.replay()
+        torch.cuda.synchronize()
+        for x, w in zip((m.out_p, m.out_d, m.lse_d), want):
+            assert torch.equal(x, w)
+            x.zero_()

@@ -428,6 +428,19 @@ def _prefill_workspace_size(device, *shape):
     return int(_lib.load().tmopt_attn_prefill_workspace_size(*shape))
 
 
+def _prefill_scratch(dev, S, max_seqlen, HQ, HKV, bts, table_wrap, window,
+                     max_context=None):
+    """Bytes of scratch of a launch that splits its keys, 0 for one launch
+    (bts: row width of the block table, 0 without one)."""
+    if bts and max_context is not None and not _prefill_workspace_size(
+            dev.index, S, max_seqlen, HQ, HKV,
+            max(1, -(-(int(max_context) - max_seqlen) // PAGE_SIZE)), 0,
+            window):
+        return 0
+    return _prefill_workspace_size(dev.index, S, max_seqlen, HQ, HKV, bts,
+                                   table_wrap, window)
+
+
 def prefill_varlen(q, k, v, cu_seqlens, scale, window=0, max_seqlen=None,
                    prior_lens=None, k_pool=None, v_pool=None,
                    block_table=None, table_wrap=0, rel=None, out=None,
@@ -477,9 +490,10 @@ def prefill_varlen(q, k, v, cu_seqlens, scale, window=0, max_seqlen=None,
 def _prefill_varlen(q, k, v, cu_seqlens, scale, window, max_seqlen,
                     prior_lens, k_pool, v_pool, block_table, table_wrap, rel,
                     out, lse, return_lse, reject, max_context=None,
-                    split=True):
+                    split=True, workspace=None):
     """prefill_varlen; split False: one launch, for a caller that fills the
-    rest of the device with other work."""
+    rest of the device with other work; workspace: uint8 scratch of at least
+    _prefill_scratch bytes instead of an allocation."""
     total, HQ, D = q.shape
     _check_rows(q, "q")
     assert cu_seqlens.dtype == torch.int32 and cu_seqlens.dim() == 1
@@ -548,14 +562,14 @@ def _prefill_varlen(q, k, v, cu_seqlens, scale, window, max_seqlen,
     # scratch for the pieces of a launch too small for the device (0 bytes
     # for any other): the kernel splits its keys
     bts = block_table.stride(0) if pooled else 0
-    n = 0
-    if split and (max_context is None or not pooled or _prefill_workspace_size(
-            dev.index, S, int(max_seqlen), HQ, HKV,
-            max(1, -(-(int(max_context) - int(max_seqlen)) // page_size)), 0,
-            int(window))):
-        n = _prefill_workspace_size(dev.index, S, int(max_seqlen), HQ, HKV,
-                                    bts, int(table_wrap), int(window))
-    ws = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
+    n = _prefill_scratch(dev, S, int(max_seqlen), HQ, HKV, bts,
+                         int(table_wrap), int(window),
+                         max_context) if split else 0
+    ws = None
+    if n:
+        ws = workspace if workspace is not None else torch.empty(
+            n, dtype=torch.uint8, device=dev)
+        n = ws.numel()
     _lib.call("tmopt_attn_prefill_varlen_split", _ptr(q), q.stride(0),
               q.stride(1),
               _ptr(k) if own else None, *ks,

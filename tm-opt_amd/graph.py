@@ -166,6 +166,17 @@ class MixedStepGraph:
         self.lse_d = torch.empty((B, HQ), dtype=torch.float32, device=dev)
         self.ws = attn.decode_workspace(B, HQ, HKV, dev,
                                         max(self.wgs.values()))
+        # scratch of the split prefill, one for every layer (they run in
+        # order); beside the decode no compute unit is idle for split keys
+        # (two 404-token chunks, 60 decode rows, four layers 403 us in one
+        # prefill launch per layer, 422 us in two)
+        self.max_context = max(p + n for p, n in zip(step.chunk_prior,
+                                                     step.chunk_lens))
+        n = 0 if overlap else max(attn._prefill_scratch(
+            dev, self.n_chunks, self.max_chunk, HQ, HKV, t.stride(0), 0,
+            0 if g else step.window, self.max_context)
+            for t, g in zip(step.tables, step.is_global))
+        self.ws_p = torch.empty(n, dtype=torch.uint8, device=dev)
         self.min_pages = min_pages
         self.overlap = overlap
         self.side = torch.cuda.Stream(device=dev) if overlap else None
@@ -181,13 +192,11 @@ class MixedStepGraph:
                                 cu_seqlens=s.cu_all,
                                 max_seqlen=self.max_chunk)
         if "prefill" in parts:
-            # (beside the decode no compute unit is idle for split keys: two
-            # 404-token chunks, 60 decode rows, four layers 403 us in one
-            # prefill launch per layer, 422 us in two)
             attn._prefill_varlen(s.q_prefill, None, None, s.cu_chunks,
                                  s.scale, w, self.max_chunk, s.prior, kp, vp,
                                  t[:self.n_chunks], 0, None, self.out_p,
-                                 None, False, None, split=not self.overlap)
+                                 None, False, None, self.max_context,
+                                 not self.overlap, self.ws_p)
         if "decode" in parts:
             attn.decode_paged(s.q_decode, kp, vp, t[self.n_chunks:],
                               s.dec_ctx, s.scale, window=w,
