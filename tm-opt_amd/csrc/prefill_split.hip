@@ -17,16 +17,16 @@ __global__ __launch_bounds__(512) void prefill_split_kernel(PrefillArgs a) {
   constexpr int BQ = 256 / REP;
   const int lane = threadIdx.x & 63;
   const int level = (int)blockIdx.x / a.n_base;
-  const int item = (int)blockIdx.x - level * a.n_base;
-  const Work wk = schedule(a, BQ, lane, item);
+  const Work wk = schedule(a, BQ, lane, (int)blockIdx.x - level * a.n_base);
+  const bool first = level == 0 && threadIdx.x == 0;
   if (wk.seq < 0) {
-    if (level == 0 && threadIdx.x == 0) a.part_n[item] = 0;
+    if (first) a.part_n[blockIdx.x] = 0;
     return;
   }
   const Tiles tl = item_tiles(a, BQ, wk.prior, wk.len, wk.qb);
   const Pieces pc = key_pieces(a, BQ, lane, wk, tl);
   if (level >= pc.nall) return;
-  if (level == 0 && threadIdx.x == 0) a.part_n[item] = pc.nall;
+  if (first) a.part_n[blockIdx.x] = pc.nall;
   const int t0 = pc.begin(level, tl.n), t1 = pc.begin(level + 1, tl.n);
   const int slot = pc.nall > 1 ? (int)blockIdx.x : -1;
   if constexpr (REL) {
