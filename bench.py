@@ -552,7 +552,7 @@ def bench_prefill_append(tm, compat, sets, window, HKV, steps, warmup):
 
     def separate(a):
         cs = caches(order[id(a)])
-        compat._append_rows(compat._kv_rows(a[1]), compat._kv_rows(a[2]), cs,
+        compat._append_rows(*compat._kv_pair(a[1], a[2]), cs,
                             [T] * Bp)
         compat.attn_prefill_fused(*a)
 
@@ -561,7 +561,7 @@ def bench_prefill_append(tm, compat, sets, window, HKV, steps, warmup):
 
     def packed(a):
         cs = caches(order[id(a)])
-        kr, vr = compat._kv_rows(a[1]), compat._kv_rows(a[2])
+        kr, vr = compat._kv_pair(a[1], a[2])
         compat._append_rows(kr, vr, cs, [T] * Bp)
         kt = kr.contiguous().transpose(1, 2)     # token-major copies
         vt = vr.contiguous().transpose(1, 2)

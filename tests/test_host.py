@@ -15,19 +15,19 @@ def _cm(B, HK, T, D=128):
 
 @pytest.mark.parametrize("B,T", [(1, 8), (3, 200), (6, 1536), (2, 16)])
 def test_kv_rows_reads_channel_major_in_place(B, T):
-    """compat._kv_rows hands channel-major K/V with 16-byte aligned dim rows
+    """compat._kv_pair hands channel-major K/V with 16-byte aligned dim rows
     (T % 8 == 0) to the kernels as a view of the same memory: run stride =
     batch stride, token stride 1, dim stride T (what the prefill's
     channel-major source and the KV write read in place)."""
     compat = import_module("tm-opt_amd.compat")
     HK, D = 4, 128
-    k = _cm(B, HK, T, D)
-    r = compat._kv_rows(k)
-    assert r.shape == (B, T, HK, D)
-    assert r.data_ptr() == k.data_ptr()
-    assert r.stride()[1:] == (1, D * T, T)
-    assert r.stride(0) % 8 == 0 and (B == 1 or r.stride(0) == HK * D * T)
-    assert torch.equal(r, k.transpose(1, 2))
+    k, v = _cm(B, HK, T, D), _cm(B, HK, T, D)
+    for x, r in zip((k, v), compat._kv_pair(k, v)):
+        assert r.shape == (B, T, HK, D)
+        assert r.data_ptr() == x.data_ptr()
+        assert r.stride()[1:] == (1, D * T, T)
+        assert r.stride(0) % 8 == 0 and (B == 1 or r.stride(0) == HK * D * T)
+        assert torch.equal(r, x.transpose(1, 2))
 
 
 @pytest.mark.parametrize("B,T", [(3, 77), (1, 5), (2, 100)])
@@ -40,9 +40,15 @@ def test_kv_rows_copies_unaligned_channel_major(B, T):
     HK, D = 2, 128
     x = torch.randn((B, HK * D, T), generator=g).to(torch.bfloat16)
     k = x.transpose(1, 2).view(B, T, HK, D).transpose(1, 2)
-    r = compat._kv_rows(k)
-    assert r.data_ptr() != k.data_ptr() and r.is_contiguous()
-    assert torch.equal(r, k.transpose(1, 2))
+    v = torch.flip(x, (0,)).transpose(1, 2).view(B, T, HK, D).transpose(1, 2)
+    even = _cm(B, HK, 8 * T, D)[:, :, :T]
+    for a, b in ((k, v), (even, v), (k, even)):
+        for x, r in zip((a, b), compat._kv_pair(a, b)):
+            if x is even:                    # one of the two in place
+                assert r.data_ptr() == x.data_ptr()
+            else:
+                assert r.data_ptr() != x.data_ptr() and r.is_contiguous()
+            assert torch.equal(r, x.transpose(1, 2))
 
 
 def test_kv_rows_token_major_views():
@@ -54,12 +60,12 @@ def test_kv_rows_token_major_views():
     a = torch.zeros((B, T, HK, D), dtype=torch.bfloat16).transpose(1, 2)
     b = torch.zeros((B, HK, T, D), dtype=torch.bfloat16)
     for x in (a, b):
-        r = compat._kv_rows(x)
-        assert r.data_ptr() == x.data_ptr() and r.stride(3) == 1
+        for r in compat._kv_pair(x, x):
+            assert r.data_ptr() == x.data_ptr() and r.stride(3) == 1
     one = torch.zeros((HK * D * 8 + 4,), dtype=torch.bfloat16)[:HK * D * 8]
     one = one.as_strided((1, HK, 8, D), (3, D * 8, 1, 8))
-    r = compat._kv_rows(one)
-    assert r.data_ptr() == one.data_ptr() and r.stride(0) % 8 == 0
+    for r in compat._kv_pair(one, one):
+        assert r.data_ptr() == one.data_ptr() and r.stride(0) % 8 == 0
 
 
 def test_c3_lengths_cover_the_window_edges():

@@ -137,19 +137,12 @@ def _in_place(x):
     return xt, aligned and (token_major or channel_major)
 
 
-def _kv_rows(x):
-    """[B, HK, T, D] K or V (any strides) -> a [B, T, HK, D] view that the
-    prefill and the KV write both read in place (see _in_place). Anything else
-    (e.g. channel-major with T % 8 != 0) becomes a token-major copy, so a
-    caller can rely on both kernels accepting the result before it changes any
-    cache."""
-    xt, ok = _in_place(x)
-    return xt if ok else xt.contiguous()
-
-
 def _kv_pair(k, v):
-    """_kv_rows of K and V. Channel-major rows that neither kernel reads in
-    place (the sconv output at T % 8 != 0) are laid out in one launch."""
+    """[B, HK, T, D] K and V (any strides) -> [B, T, HK, D] views that the
+    prefill and the KV write both read in place (see _in_place). Anything else
+    becomes a token-major copy, so a caller can rely on both kernels accepting
+    the result before it changes any cache: channel-major rows (the sconv
+    output at T % 8 != 0) of both in one launch."""
     (kt, k_ok), (vt, v_ok) = _in_place(k), _in_place(v)
     if (not k_ok and not v_ok and k.is_cuda and kt.stride(1) == 1 and
             vt.stride(1) == 1 and kt.shape[3] == attn.HEAD_DIM and
@@ -209,7 +202,7 @@ def _append_rows(k, v, caches, lens):
     """The prefill's cache population (model.py:507-512:
     st.cache.append(kn[i, :lens[i]], vv[i, :lens[i]])) done natively: each
     row's K/V [lens[i], HK, D] is appended to its cache straight from the
-    [B, T, HK, D] rows of _kv_rows (channel-major or token-major, a layout
+    [B, T, HK, D] rows of _kv_pair (channel-major or token-major, a layout
     the write kernels accept, checked before any cache changes), pages
     allocated on the host as
     PagedKV.append does (kv.py:196-198), ring rows as RingKV.append keeps
