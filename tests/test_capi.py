@@ -155,6 +155,87 @@ def test_invalid_arguments_return_status(tm):
     assert b"T must be positive" in lib.tmopt_last_error()
 
 
+def test_preparing_and_flat_entries_refuse(tm):
+    """The launches that prepare a call and the flat decode: sizes outside
+    their ranges, null and misaligned pointers, and no-ops."""
+    lib, e = tm._lib.load(), tm._lib
+    null, p, odd = (ctypes.c_void_p(x) for x in (0, 16, 17))
+
+    def pack(k=p, out=p, B=1, T=5, HKV=2, D=128):
+        return lib.tmopt_pack_rows(k, 1280, 640, 5, p, 1280, 640, 5, B, T,
+                                   HKV, D, out, p, null)
+    assert pack(B=0) == pack(T=0) == 0
+    for kw in (dict(B=-1), dict(B=65536), dict(T=-1), dict(HKV=0),
+               dict(HKV=32768), dict(k=null), dict(out=null), dict(k=odd),
+               dict(out=ctypes.c_void_p(24))):
+        assert pack(**kw) == e.TMOPT_EINVAL, kw
+    assert pack(D=64) == e.TMOPT_EUNSUPPORTED
+
+    def tables(td=p, stride=8, rows=3, slots=p, ns=2, prior=p, npr=2, width=8,
+               table=p, start=p):
+        return lib.tmopt_chunk_tables(td, stride, rows, slots, ns, prior, npr,
+                                      width, table, start, null, 0, null,
+                                      null)
+    assert tables(ns=0, npr=0, slots=null, prior=null, table=null,
+                  start=null) == 0
+    for kw in (dict(ns=-1), dict(ns=65536), dict(npr=65536), dict(width=0),
+               dict(slots=null), dict(table=null), dict(prior=null),
+               dict(start=null), dict(rows=0), dict(stride=7)):
+        assert tables(**kw) == e.TMOPT_EINVAL, kw
+
+    def flat(q=p, rows=p, pos=p, Lg=100, B=1, HQ=32, HKV=4, D=128, ps=16,
+             pages=1, min_pages=8, nbytes=1 << 30):
+        return lib.tmopt_attn_decode_flat(q, p, p, rows, Lg, pos, B, HQ, HKV,
+                                          D, ps, pages, 0.1, null, 0,
+                                          min_pages, 0, p, null, p, nbytes,
+                                          null)
+    assert flat(B=0, q=null) == 0
+    for kw in (dict(B=-1), dict(q=null), dict(q=odd), dict(rows=null),
+               dict(pos=null), dict(Lg=0), dict(HQ=33), dict(pages=0),
+               dict(min_pages=0)):
+        assert flat(**kw) == e.TMOPT_EINVAL, kw
+    for kw in (dict(B=8193), dict(D=64), dict(ps=32)):
+        assert flat(**kw) == e.TMOPT_EUNSUPPORTED, kw
+    assert flat(nbytes=64) == e.TMOPT_EWORKSPACE
+
+
+def test_split_prefill_refuses_what_the_prefill_does(tm):
+    """tmopt_attn_prefill_varlen_split takes and refuses the same arguments as
+    tmopt_attn_prefill_varlen, with a workspace or without, plus one that is
+    short or misaligned; the size is 0 where nothing can be launched."""
+    lib, e = tm._lib.load(), tm._lib
+    null, p = ctypes.c_void_p(0), ctypes.c_void_p(16)
+    size = lib.tmopt_attn_prefill_workspace_size
+    need = size(1, 64, 32, 4, 500, 0, 0)
+    assert need > 0
+    # at most 2 x 129 KB per compute unit (256 where no device answers) and a
+    # count per block
+    most = max(size(S, n, 32, 4, 4000, 0, 0) for S in (1, 2, 3, 5)
+               for n in (1, 33, 64, 200, 500))
+    assert most <= 512 * 129 * 1024 + 4096
+    for bad in ((0, 64, 32, 4), (1, 0, 32, 4), (-1, 64, 32, 4),
+                (1, 64, 0, 4), (1, 64, 32, 0), (1, 64, 33, 4)):
+        assert size(*bad, 500, 0, 0) == 0
+
+    def call(split, S=1, n=64, HQ=32, HKV=4, D=128, scale=0.1, window=0,
+             table=p, pages=100, ps=16, q=p, ws=p, nbytes=1 << 30):
+        a = [q, 4096, 128, null, 0, 0, 0, 1, null, 0, 0, 0, 1, p, p, S, n, p,
+             p, table, 500, 0, ps, pages, HQ, HKV, D, window, scale, null, 0,
+             0, 0, p, 4096, 128, null, null]
+        if not split:
+            return lib.tmopt_attn_prefill_varlen(*a, null)
+        return lib.tmopt_attn_prefill_varlen_split(*a, ws, nbytes, null)
+    for kw in (dict(S=-1), dict(S=65536), dict(n=-1), dict(HQ=33),
+               dict(D=64), dict(scale=0.0), dict(window=-1), dict(pages=0),
+               dict(ps=32), dict(q=null), dict(table=null)):
+        want = call(False, **kw)
+        assert want in (e.TMOPT_EINVAL, e.TMOPT_EUNSUPPORTED), kw
+        assert call(True, **kw) == call(True, ws=null, nbytes=0, **kw) == want
+    assert call(True, S=0) == call(True, n=0) == 0
+    assert call(True, nbytes=need - 1) == e.TMOPT_EWORKSPACE
+    assert call(True, ws=ctypes.c_void_p(8)) == e.TMOPT_EWORKSPACE
+
+
 def test_python_wrapper_asserts_before_launch(tm):
     """The reference wrappers assert dtype/contiguity before launching
     (attn_swa.py:128-132); so do ours (no device needed to trip them)."""
