@@ -431,8 +431,8 @@ int tmopt_attn_prefill_varlen(
 
 /*
  * The same with the keys of a query block split over several work-groups
- * where the launch has fewer query blocks than the device compute units (a
- * short chunk after a long cached context, a few short prompts): a second
+ * where the launch has at most half as many query blocks as the device has
+ * compute units, and these may see many keys (a short chunk after a long cached context, a few short prompts): a second
  * launch then merges the pieces, in a fixed order. workspace: device scratch
  * of tmopt_attn_prefill_workspace_size bytes, 16-byte aligned, which needs no
  * initialisation (TMOPT_EWORKSPACE if smaller; NULL, or a size of 0: one

@@ -74,13 +74,13 @@ def test_bias_rows_at_every_alignment(tm, dev, hq, hkv, E):
 
 
 @pytest.mark.parametrize("B,hq,hkv,pages", [
-    (1, 32, 4, 500), (1, 7, 1, 33), (2, 9, 3, 400), (5, 16, 2, 90),
+    (1, 32, 4, 190), (1, 32, 4, 500), (1, 7, 1, 33), (2, 9, 3, 400), (5, 16, 2, 90),
     (23, 32, 4, 40), (24, 32, 4, 40), (64, 8, 8, 12)])
 def test_merge_shapes(tm, dev, B, hq, hkv, pages):
-    """One piece per page (min_pages 1) over grids of 1 to 200 work-groups:
-    from a merge of 192 pieces by 32 groups per head to one of two pieces, an
-    odd number of heads per work-group, more groups than pieces, sequences
-    that need no merge beside ones that do."""
+    """Shares of one page and more (min_pages 1) over grids of 7 to 200
+    work-groups: from a merge of 190 pieces, one per page, by 32 groups per
+    head to one of two pieces, an odd number of heads per work-group, more
+    groups than pieces, sequences that need no merge beside ones that do."""
     wl = import_module("tm-opt_amd.workloads")
     g = torch.Generator().manual_seed(B)
     ctx = torch.randint(1, 16 * pages, (B,), generator=g)

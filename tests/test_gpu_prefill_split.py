@@ -1,6 +1,6 @@
-"""Prefill launches of fewer query blocks than the device has compute units
-split their keys over work-groups and merge the pieces: against the fp32
-oracle, over the key sources, at the edges of pieces, bands and windows."""
+"""Prefill launches of at most half as many query blocks as the device has
+compute units split their keys over work-groups and merge the pieces: against
+the fp32 oracle, over the key sources, at the edges of pieces, bands and windows."""
 from importlib import import_module
 
 import pytest
@@ -99,7 +99,7 @@ def test_ring_chunk(tm, dev, W, prior):
 def test_split_repeats_bitwise_and_matches_one_launch(tm, dev):
     """The merge order is fixed; the unsplit entry point (no workspace) gives
     the same result to the rounding of one bf16 store. A launch of more
-    items than compute units does not split; a short workspace is refused;
+    items than half the compute units does not split; a short workspace is refused;
     a rejected launch is NaN whole."""
     wl = import_module("tm-opt_amd.workloads")
     a = _runs([130], [2500], 32, 4, 63, "paged", wl)

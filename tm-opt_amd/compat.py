@@ -57,9 +57,9 @@ def _ring_grid(B, HKV, dev):
     compute unit, need no merge launch and balance when the rings are full,
     but stream fast only on enough compute units: the line is 0.6 of them.
     Measured at W = 512, full rings, 64Q/16KV (whole rings / default grid,
-    us): B = 4 24.6 / 12.3, 32 (128 work-groups) 29.4 / 28.9, 40 (160) 32.9 /
-    34.9, 64 (256) 47.1 / 50.3, 72 (144 of two rings) 57.7 / 55.3, 80 (160)
-    58.0 / 60.4, 96 (192) 66.3 / 70.1; 32Q/4KV, B = 64 (64) 29.1 / 21.7."""
+    us): B = 4 20.8 / 13.3, 32 (128 work-groups) 27.9 / 27.3, 40 (160) 30.0 /
+    33.0, 64 (256) 43.6 / 47.0, 72 (144 of two rings) 53.5 / 54.3, 80 (160)
+    55.7 / 58.1, 96 (192) 62.2 / 63.9; 32Q/4KV, B = 64 (64) 26.2 / 19.4."""
     groups = max(1, HKV // 4)
     cus = _cus(dev.index)
     per_group = max(1, cus // groups)

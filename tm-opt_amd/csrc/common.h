@@ -87,9 +87,6 @@ as_const(const T* p) {
   return (const __attribute__((address_space(4))) T*)p;
 }
 
-// Order LDS accesses of one wave: every lane's prior LDS writes are visible
-// to every lane's later LDS reads, and the compiler may not move LDS traffic
-// across this point.
 // ---- LDS access by 32-bit LDS byte address -------------------------------
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
@@ -203,6 +200,9 @@ __device__ __forceinline__ void wait_vm() {
                              (15 << 8));
 }
 
+// Order LDS accesses of one wave: every lane's prior LDS writes are visible
+// to every lane's later LDS reads, and the compiler may not move LDS traffic
+// across this point.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

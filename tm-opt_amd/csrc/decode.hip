@@ -114,9 +114,9 @@ struct DecodeArgs {
   float* part_o;     // [B + G, HQ, D] fp32
   float* part_lse;   // [B + G, HQ]
   int* geo;          // [B + 2]: C, then the page-stream prefix pref[0..B]
+  int ids_off;       // LDS byte offset of the range's page ids
   // read by the REP 0 kernels only (any other REP implies rep == REP,
   // kv_div == 1, HKV_stored == HKV)
-  int ids_off;       // LDS byte offset of the range's page ids
   int rep;           // query heads per scheduled KV head (1..16)
   int kv_div;        // scheduled KV heads per stored one: 1 unless HQ/HKV
                      // is above 16 (then kv_div groups of `rep` query
@@ -610,12 +610,14 @@ void decode_kernel(DecodeArgs a) {
   // compute unit streams: page rows do not pass through registers, V^T is
   // read under the softmax, the next step's scalar work goes under the K
   // reads, and steps whose 32 tokens are all visible skip the masks. Measured
-  // per step of 32 keys and 4 KV heads with its data in cache: 1.40 us for the
-  // form that loaded page rows into registers one step ahead, looked up page
-  // ids step by step and zeroed, masked and rescaled on every step (2.2 us
-  // with the bias, then 8 two-byte loads per lane); here 1.05 us (1.1 us), of
-  // which the chain is 0.66 us: the loads of one compute unit, 62 GB/s, now
-  // bound it. attn_swa at B = 4, 64Q/16KV (one ring per work-group): 37.3 ->
+  // per step of 32 keys and 4 KV heads, one work-group: 1.60 us with its pages
+  // in the L2 and from HBM alike for the form that loaded page rows into
+  // registers one step ahead, looked up page ids step by step and zeroed,
+  // masked and rescaled on every step (1.86 us with the bias, then 8 two-byte
+  // loads per lane); here 0.65 us in the L2 (the chain; 1.12 us with the bias)
+  // and 1.06 us from HBM: the loads of one compute unit, 62 GB/s (41 before),
+  // now bound it. Among 128 work-groups one streams 46 GB/s (39 before), among
+  // 192 the HBM's share, 36. attn_swa at B = 4, 64Q/16KV (one ring per work-group): 37.3 ->
   // 24.6 us; B = 96: 72.6 -> 65.3 us.
   // Queries: those of the next step, if it starts a piece, go out at the top
   // of this one.
@@ -779,8 +781,11 @@ void decode_kernel(DecodeArgs a) {
 // pieces s, s + S, ..., eight pieces' loads in flight at a time; the S results
 // then merge through LDS in group order. The load latency, not the bytes, is
 // what this kernel waits on: S is chosen so that the pieces of an average
-// sequence take one round (one 50,000-token sequence cut into 185 pieces:
-// 19.3 us with S = 1, 24 rounds in a chain, 5.0 us with S = 32).
+// sequence take one round (one 50,001-token sequence cut into 184 pieces:
+// 19.3 us with S = 1, 23 rounds in a chain, 5.0 us with S = 32). A long sequence
+// among many short ones still merges in a chain, since the host knows the
+// average alone (50,001 tokens beside 31 sequences of 300: 42.6 us a call,
+// alone 26.0).
 template <int H, int S>
 __global__ __launch_bounds__(32 * H * S) void decode_combine_kernel(
     DecodeArgs a) {
@@ -873,9 +878,10 @@ void launch_combine(const DecodeArgs& a, int G, hipStream_t st) {
 
 int waves_per_wg(int HKV) { return HKV % 4 == 0 ? 4 : (HKV % 2 == 0 ? 2 : 1); }
 
-// Three work-groups per four CUs (one wave per SIMD where they run):
-// measured on MI355X, C2 / C3 decode stream fastest between 0.75 and 0.85
-// work-groups per CU, 3-8 % ahead of one per CU and 10-20 % ahead of two.
+// Three work-groups per four CUs (one wave per SIMD where they run). 160 / 176
+// / 192 / 208 / 256 / 512 work-groups, us: 64 sequences of 1K-8K (32Q/4KV) 98.8
+// / 96.7 / 96.5 / 96.7 / 99.0 / 110.5, window 4096 at 128 sequences 168.9 /
+// 164.6 / 165.1 / 166.2 / 170.7 / 178.5.
 int default_wgs(int HKV) {
   const int ny = HKV / waves_per_wg(HKV);
   const int g = 3 * device_cus() / (4 * ny);

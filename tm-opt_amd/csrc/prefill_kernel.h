@@ -254,9 +254,9 @@ __device__ __forceinline__ Tiles item_tiles(const PrefillArgs& a, int BQ,
 // 2.5-2.9): either the band is a share of its own, or the last plain piece is
 // shorter by the band's time, and the band's piece, dispatched after all the
 // others, takes its compute unit when it ends.
-// Measured (per call of the chunk adapters, bias extent 1024): 64 tokens after
-// 30,000 957 -> 131 us, 1000 after 20,000 677 -> 232 us, 500 after 15,000
-// 525 -> 320 us, 200 + 200 after 8,000 272 -> 107 us.
+// Measured (per call of the chunk adapter, 64Q/8KV, bias extent 1024): 64
+// tokens after 30,000 958 -> 96 us, 500 after 15,000 531 -> 277 us, 200 + 200
+// after 8,000 276 -> 158 us, 64 after 1,500 105 -> 43 us.
 constexpr int kMinPiece = 8;
 constexpr int kMinSplit = 16;   // tiles: two pieces
 struct Pieces {

@@ -141,11 +141,12 @@ class MixedStepGraph:
     takes two thirds of its stand-alone size (half the compute units) and a
     window layer's its stand-alone size (it is done in about half the time
     of that layer's prefill and then leaves the prefill every unit).
-    Measured on config 5 (one box, four alternating runs each): 31.4-31.6
-    ms per step, against 31.8-32.8 ms with two thirds for both kinds; with
-    two thirds for both on another box 30.6 ms, against 31.4 ms with the
-    stand-alone grid for both and 31.7 ms without the second stream.
-    num_workgroups > 0 sets one grid for both kinds."""
+    Measured on four layers (one of them global) of a step of two 2048-token
+    chunks and 96 decode rows (work-groups on global / window layers, us):
+    128 / 192, the default, 1763-1784; 64 / 192 1965, 96 / 192 1783, 112 / 192
+    1762-1787, 144 / 192 1764-1771, 160 / 192 1779-1788, 192 / 192 1841; 128 /
+    128 1824-1867, 128 / 160 1776-1785, 128 / 224 1774. num_workgroups > 0
+    sets one grid for both kinds."""
 
     def __init__(self, step, min_pages=8, num_workgroups=0, overlap=True):
         self.s = step
