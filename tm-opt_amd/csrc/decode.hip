@@ -782,7 +782,7 @@ void decode_kernel(DecodeArgs a) {
 // then merge through LDS in group order. The load latency, not the bytes, is
 // what this kernel waits on: S is chosen so that the pieces of an average
 // sequence take one round (one 50,001-token sequence cut into 184 pieces:
-// 19.3 us with S = 1, 23 rounds in a chain, 5.0 us with S = 32). A long sequence
+// 19.3 us with S = 1, 23 rounds in a chain, 5.8 us with S = 32). A long sequence
 // among many short ones still merges in a chain, since the host knows the
 // average alone (50,001 tokens beside 31 sequences of 300: 42.6 us a call,
 // alone 26.0).
