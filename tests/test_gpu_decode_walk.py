@@ -164,3 +164,25 @@ def test_merge_of_infinite_values(tm, dev, B, pages):
         out = out.cpu()
         assert torch.equal(out.isinf(), want), wgs
         assert not out.isnan().any(), wgs
+
+
+def test_merge_of_more_heads_than_a_grid_dimension(tm, dev):
+    """65,538 query heads over 64 ranges: the merge's grid holds heads in its
+    y dimension (65,536 at most), eight to a work-group. Against the launch
+    that splits nothing, to two roundings of O to bf16 (2^-7 of the value) and
+    of P (2^-9 of the values' sums)."""
+    g = torch.Generator(device=dev).manual_seed(49)
+    HQ, HKV, n = 65538, 32769, 70
+    r = lambda *s: torch.randn(s, generator=g, device=dev,  # noqa: E731
+                               dtype=torch.bfloat16)
+    q, kp, vp = r(1, HQ, 128), r(5, 16, HKV, 128), r(5, 16, HKV, 128)
+    table = torch.tensor([[3, 0, 4, 2, 1]], dtype=torch.int32, device=dev)
+    ctx = torch.tensor([n], dtype=torch.int32, device=dev)
+    one = tm.decode_paged(q, kp, vp, table, ctx, 128 ** -0.5,
+                          num_workgroups=1)
+    out = tm.decode_paged(q, kp, vp, table, ctx, 128 ** -0.5, min_pages=1,
+                          num_workgroups=64)
+    torch.cuda.synchronize()
+    assert ((one[0].float() - out[0].float()).abs() <=
+            2 ** -7 * one[0].float().abs() + 1e-2).all()
+    assert (one[1] - out[1]).abs().max() <= 1e-4

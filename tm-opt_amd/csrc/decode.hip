@@ -862,9 +862,11 @@ __global__ __launch_bounds__(32 * H * S) void decode_combine_kernel(
 }
 
 // The merge's shape, from the number of pieces of an average sequence (at most
-// one more than its share of the grid's G ranges).
+// one more than its share of the grid's G ranges). Heads per work-group times
+// the grid's y dimension (65,536 at most) must hold every head, so more of them
+// than that take the shape of eight.
 void launch_combine(const DecodeArgs& a, int G, hipStream_t st) {
-  const int np = 1 + G / a.B;
+  const int np = a.HQ > 65535 ? 1 : 1 + G / a.B;
   if (np <= 8)
     hipLaunchKernelGGL((decode_combine_kernel<8, 1>),
                        dim3(a.B, (a.HQ + 7) / 8), dim3(256), 0, st, a);
