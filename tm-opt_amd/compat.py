@@ -398,7 +398,8 @@ def attn_prefill_chunk_swa(q, k, v, rel, pool_k, pool_v, slots, prior,
     appends the chunks to the rings (only the last W positions survive).
     max_seqlen: the longest chunk; with several sequences pass it to keep
     the call free of host synchronisation (graph capture). max_context: the
-    longest prior + chunk, where the host knows it (prefill_varlen's).
+    longest prior + chunk, where the host knows it (prefill_varlen's). Few
+    queries over many keys take prefill_varlen's scratch, up to 66 MB.
     Returns out [total, H, D] bf16."""
     total, H, D = q.shape
     S1, W, HK, _ = pool_k.shape
@@ -440,7 +441,8 @@ def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
     chunk; with several sequences pass it to keep the call free of host
     synchronisation (graph capture). max_context: the longest prior + chunk,
     where the host knows it (prefill_varlen's: the page table's width says
-    nothing about it). A slot outside table_dev rejects the call on the
+    nothing about it); without it a call of few queries takes prefill_varlen's
+    scratch, up to 66 MB, whatever its context. A slot outside table_dev rejects the call on the
     device, without a host synchronisation: out is NaN, and nothing of that
     sequence is appended. Returns out [total, H, D]."""
     total, H, D = q.shape
