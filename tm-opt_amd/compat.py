@@ -442,9 +442,9 @@ def attn_prefill_chunk_global(q, k, v, rel, pool_kp, pool_vp, table_dev,
     synchronisation (graph capture). max_context: the longest prior + chunk,
     where the host knows it (prefill_varlen's: the page table's width says
     nothing about it); without it a call of few queries takes prefill_varlen's
-    scratch, up to 66 MB, whatever its context. A slot outside table_dev rejects the call on the
-    device, without a host synchronisation: out is NaN, and nothing of that
-    sequence is appended. Returns out [total, H, D]."""
+    scratch, up to 66 MB, whatever its context. A slot outside table_dev
+    rejects the call on the device, without a host synchronisation: out is NaN,
+    and nothing of that sequence is appended. Returns out [total, H, D]."""
     total, H, D = q.shape
     assert pool_kp.is_contiguous() and pool_vp.is_contiguous()
     assert pool_kp.shape[1] == PAGE
