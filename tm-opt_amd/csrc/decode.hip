@@ -864,15 +864,19 @@ __global__ __launch_bounds__(32 * H * S) void decode_combine_kernel(
 // The merge's shape, from the number of pieces of an average sequence (at most
 // one more than its share of the grid's G ranges). Heads per work-group times
 // the grid's y dimension (65,536 at most) must hold every head, so more of them
-// than that take the shape of eight.
+// than that take the shape of eight. Groups of lanes per head cost waves, which
+// a prefill beside the decode makes wait: with 1 / 4 / 8 of them, us, 32Q/4KV, 4
+// sequences of 4K-8K 20.0 / 16.5 / 16.5, 9 up to 4.7K 17.9 / 16.6 / 17.2, 20 of
+// 4K-8K 43.4 / 43.5 / 44.9; a mixed step (four layers, two 1285-token chunks, 9
+// decode rows) 445.8 / 448.0 / 453.8, against 452.1 before the merge had groups.
 void launch_combine(const DecodeArgs& a, int G, hipStream_t st) {
   const int np = a.HQ > 65535 ? 1 : 1 + G / a.B;
   if (np <= 8)
     hipLaunchKernelGGL((decode_combine_kernel<8, 1>),
                        dim3(a.B, (a.HQ + 7) / 8), dim3(256), 0, st, a);
   else if (np <= 64)
-    hipLaunchKernelGGL((decode_combine_kernel<2, 8>),
-                       dim3(a.B, (a.HQ + 1) / 2), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((decode_combine_kernel<2, 4>),
+                       dim3(a.B, (a.HQ + 1) / 2), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL((decode_combine_kernel<1, 32>), dim3(a.B, a.HQ),
                        dim3(1024), 0, st, a);
